@@ -2,8 +2,8 @@
 //
 // Every product is one "NT" form, C[i,j] = sum_k A[i,k] B[j,k] with both
 // operands row-major along k, computed with v_mfma_f32_32x32x16_{f16,bf16}
-// (fp32 accumulation) from LDS-staged k tiles (64 deep; 32 deep where k is an
-// odd multiple of 32). The epilogue forms
+// (fp32 accumulation, every element over k in order, whatever the tile) from
+// LDS-staged k tiles (64 deep; 32 deep where k is an odd multiple of 32). The epilogue forms
 // alpha * acc + beta * D[i,j] and rounds once to the storage type; in mode
 // kOutRoundAcc it rounds the product to the storage type first, then forms
 // alpha * bf16(acc) + beta * D and rounds again (a product stored by one
@@ -30,6 +30,7 @@
 #include <mutex>
 #include <vector>
 #include <algorithm>
+#include <type_traits>
 
 namespace dionw {
 namespace {
@@ -306,18 +307,17 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_nt_kernel(GemmArgs g) {
 
 // ---- pipelined tile kernels ----------------------------------------------------
 //
-// Two tile shapes (PipeCfg): 256x256 per workgroup of 16 waves (4x4, 64x64 per
-// wave: 4 accumulators of 32x32) and 128x128 per workgroup of 4 waves (2x2,
-// 64x64 per wave, two workgroups per CU). k advances through an LDS ring filled
-// by direct-to-LDS loads (global_load_lds_dwordx4): two 64-deep stages when k
-// is a multiple of 64, four 32-deep stages when it is an odd multiple of 32; a
-// stage is requested one stage (64-deep) or three stages (32-deep) before it is
-// consumed. Waits are explicit: before a stage is read every wave waits for its
-// own loads of it (vmcnt) and for its reads of the stage about to be refilled
-// (lgkmcnt), then the workgroup meets at one barrier. Rows beyond m / n load a
-// clamped valid row (only outputs that are never stored see them), so every
-// wave issues the same number of loads per stage and the vmcnt arithmetic is
-// exact; k must be a multiple of 32.
+// For the products that the quadrant tiles below do not take (depths that are an
+// odd multiple of 32, or 64; an addend whose rows are not 16-byte chunks; operands
+// past 2 GB): 256x256 per workgroup of 16 waves (4x4, 64x64 per wave) or 128x128
+// per workgroup of 4 waves (2x2, two workgroups per CU). k advances through an LDS
+// ring of four 32-deep stages filled by direct-to-LDS loads, a stage requested
+// three stages before it is consumed. Waits are explicit: before a stage is read
+// every wave waits for its own loads of it (vmcnt) and for its reads of the stage
+// about to be refilled (lgkmcnt), then the workgroup meets at one barrier. Rows
+// beyond m / n load a clamped valid row (only outputs that are never stored see
+// them), so every wave issues the same number of loads per stage and the vmcnt
+// arithmetic is exact; k must be a multiple of 32.
 
 // Tile configuration: BM x BN output tile, WM x WN waves, STAGES-deep LDS ring of
 // BK-deep stages.
@@ -362,10 +362,12 @@ constexpr int epi_ld() { return BN + 8; }
 template <int BM, int BN>
 constexpr size_t epi_lds_bytes() { return (size_t)BM * epi_ld<BN>() * 2; }
 
-template <typename T, typename OUT_T, int MODE, int NT, int BM, int BN, int FM, int FN>
+// frow(i) / fcol(j): the tile row / column where the wave's fragment row i / column j starts.
+template <typename T, typename OUT_T, int MODE, int NT, int BM, int BN, int FM, int FN,
+          typename FROW, typename FCOL>
 __device__ __forceinline__ void staged_epilogue(const GemmArgs& g, f32x16 (&acc)[FM][FN],
-                                                int64_t bidx, int m0, int n0, int wrow0,
-                                                int wcol0, bool diag_tile, unsigned char* smem) {
+                                                int64_t bidx, int m0, int n0, FROW frow,
+                                                FCOL fcol, bool diag_tile, unsigned char* smem) {
   constexpr int ELD = epi_ld<BN>();
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   const int tid = threadIdx.x, lane = tid & 63, lrow = lane & 31, lk = lane >> 5;
@@ -421,16 +423,16 @@ __device__ __forceinline__ void staged_epilogue(const GemmArgs& g, f32x16 (&acc)
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
-        const int col = wcol0 + j * 32 + lrow;
+        const int col = fcol(j) + lrow;
         float dval[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const int row = wrow0 + i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3);
+          const int row = frow(i) + 8 * (e >> 2) + 4 * lk + (e & 3);
           dval[e] = (float)reinterpret_cast<const T*>(tile)[row * ELD + col];
         }
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const int row = wrow0 + i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3);
+          const int row = frow(i) + 8 * (e >> 2) + 4 * lk + (e & 3);
           tile[row * ELD + col] = round_out<OUT_T, MODE>(
               axpby(g.alpha, product_value<OUT_T, MODE>(acc[i][j][e]), g.beta, dval[e]));
         }
@@ -440,10 +442,10 @@ __device__ __forceinline__ void staged_epilogue(const GemmArgs& g, f32x16 (&acc)
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
-        const int col = wcol0 + j * 32 + lrow;
+        const int col = fcol(j) + lrow;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const int row = wrow0 + i * 32 + 8 * (e >> 2) + 4 * lk + (e & 3);
+          const int row = frow(i) + 8 * (e >> 2) + 4 * lk + (e & 3);
           tile[row * ELD + col] =
               round_out<OUT_T, MODE>(g.alpha * product_value<OUT_T, MODE>(acc[i][j][e]));
         }
@@ -534,6 +536,12 @@ template <int N>
 __device__ __forceinline__ void wait_vm_lgkm0() {
   // s_waitcnt vmcnt(N) expcnt(7) lgkmcnt(0)
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
+}
+
+// s_waitcnt vmcnt(N) lgkmcnt(R): N loads and the last R LDS reads may be in flight.
+template <int N, int R>
+__device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (R << 8) | ((N >> 4) << 14));
 }
 
 typedef short v4i16 __attribute__((ext_vector_type(4)));
@@ -698,7 +706,496 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
   }
 
   staged_epilogue<T, OUT_T, MODE, CFG::threads, PBM, PBN, FM, FN>(
-      g, acc, bidx, m0, n0, wm * WTM, wn * WTN, diag_tile, smem);
+      g, acc, bidx, m0, n0, [&](int i) { return wm * WTM + i * 32; },
+      [&](int j) { return wn * WTN + j * 32; }, diag_tile, smem);
+}
+
+
+// ---- tiles in quadrants ------------------------------------------------------------
+//
+// The products' main kernel, for depths that are a multiple of 64. WM x WN waves;
+// the tile is 2 WM FI 32 rows by 2 WN FJ 32 columns, split into two halves each
+// way. A wave owns FI x FJ fragments of 32x32 in each of the four quadrants (rows
+// half qi, columns half qj) and multiplies them one after the other, 0 0, 0 1,
+// 1 1, 1 0: each step changes one operand's half, whose fragments are read from
+// LDS under the MFMAs of the step before, into registers that those MFMAs free
+// k-step by k-step. So the MFMAs wait for no LDS read.
+//
+// An operand's half stage (64 deep) is a slot of its own in a ring of two stages.
+// Its fragments leave LDS early (whole-depth fragments sit in registers), so the
+// slot is refilled two stages ahead while the rest of its stage is still in use:
+// a load has a whole stage (four quadrants) or more to land, and the workgroup
+// meets at two barriers per stage. Loads are direct to LDS through buffer
+// resources (a scalar stage offset plus a lane offset: no address arithmetic in
+// the loop, and only vmcnt counts them, so waits for LDS reads stay partial).
+// The last two stages leave their slots to the addend's tile, laid out as the
+// epilogue reads it. Quadrants that store nothing (past a ragged side, below the
+// diagonal of a symmetric product's diagonal tile) are not multiplied.
+//
+// MFMAs take the column operand first, so that a lane holds 4 consecutive columns
+// of a row: the epilogue moves 8 bytes per LDS access, and the mirrored store
+// reads its columns with transpose reads.
+//
+// What bounds it: the MFMA pipe and the board's power limit. At 8192^3 the pipe is
+// busy 80% of cycles (62% with one barrier per stage and every stage's loads
+// waited for one stage later, 16 waves of 64x64), at 1.36-1.5 GHz. Measured, before
+// and after, us: 8192^3 1015 / 890; 8 x 3584^3 symmetric with addend 457 / 398
+// (806 / 924 TFLOP/s); 4 x 3584 x 4096 x 3584 438 / 382; 16 x 1024^3 symmetric with
+// addend 38 / 32; 64 x 1408 x 1408 x 2048 389 / 324 (whose ragged tiles multiply
+// half). Not kept: four waves of 128x128 (442 on 8 x 3584^3 where this took 421),
+// a barrier per quadrant (421 against 398), the loads after later k-steps (+1%).
+template <int WM_, int WN_, int FI_, int FJ_>
+struct QuadCfg {
+  static constexpr int WM = WM_, WN = WN_, FI = FI_, FJ = FJ_;
+  static constexpr int waves = WM * WN, threads = waves * 64;
+  static constexpr int HM = WM * FI * 32, HN = WN * FJ * 32;  // half tile rows / columns
+  static constexpr int BM = 2 * HM, BN = 2 * HN;
+  static constexpr int depth = 64;
+  static constexpr int a_half = HM * depth, b_half = HN * depth;   // elements of a half stage
+  static constexpr int LA = a_half / 8 / threads, LB = b_half / 8 / threads;  // loads per lane
+  static constexpr size_t lds_bytes = (size_t)2 * 2 * (a_half + b_half) * 2;
+  static_assert(LA == LB && LA >= 1, "both operands' halves take the same number of loads");
+  static_assert((size_t)BM * BN * 2 <= lds_bytes, "the output tile is assembled in the ring");
+};
+
+using BigTile = QuadCfg<2, 4, 2, 1>;  // 256x256, 8 waves, one workgroup per CU
+using MidTile = QuadCfg<2, 2, 1, 1>;  // 128x128, 4 waves, two workgroups per CU
+
+// The output tile in LDS: rows of BN elements, 16-byte chunk ch of row r at
+// ch ^ epi_swz(r).
+__device__ __forceinline__ int epi_swz(int r) { return ((r & 3) << 1) | ((r >> 2) & 1) | (r & 8); }
+template <int BN>
+__device__ __forceinline__ int epi_off(int r, int ch) { return r * BN + ((ch ^ epi_swz(r)) << 3); }
+
+template <typename T, typename OUT_T, int MODE, typename CFG, bool ADD>
+__device__ __forceinline__ void quad_epilogue(const GemmArgs& g, f32x16 (&acc)[2 * CFG::FI][2 * CFG::FJ],
+                                              int64_t bidx, int m0, int n0, int wave, int lane,
+                                              bool skip1x, bool skipx1, bool diag_tile,
+                                              unsigned char* smem) {
+  constexpr int BM = CFG::BM, BN = CFG::BN, NT = CFG::threads, CH = BN / 8;
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  typedef OUT_T o4 __attribute__((ext_vector_type(4)));
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  const int wm = wave / CFG::WN, wn = wave % CFG::WN;
+  const int tid = wave * 64 + lane;
+  const int lrow = lane & 31, lk = lane >> 5;
+  OUT_T* tile = reinterpret_cast<OUT_T*>(smem);
+  OUT_T* C = g.c ? reinterpret_cast<OUT_T*>(g.c) + bidx * g.sc : nullptr;
+  OUT_T* CT = g.ct ? reinterpret_cast<OUT_T*>(g.ct) + bidx * g.sct : nullptr;
+  OUT_T* CD = g.c_diag ? reinterpret_cast<OUT_T*>(g.c_diag) + bidx * g.sc : nullptr;
+  __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt(0) lgkmcnt(0): the addend has landed
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < 2 * CFG::FI; ++i) {
+    if (i >= CFG::FI && skip1x) continue;
+#pragma unroll
+    for (int j = 0; j < 2 * CFG::FJ; ++j) {
+      if (j >= CFG::FJ && skipx1) continue;
+      if (i >= CFG::FI && j < CFG::FJ && diag_tile) continue;
+      const int r = (i / CFG::FI) * CFG::HM + (wm * CFG::FI + i % CFG::FI) * 32 + lrow;
+      const int ch0 = ((j / CFG::FJ) * CFG::HN + (wn * CFG::FJ + j % CFG::FJ) * 32) / 8;
+      t4 d[4];
+      if (ADD) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          d[q] = *reinterpret_cast<const t4*>(reinterpret_cast<const T*>(tile) +
+                                              epi_off<BN>(r, ch0 + q) + 4 * lk);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        o4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float p = product_value<OUT_T, MODE>(acc[i][j][4 * q + e]);
+          v[e] = round_out<OUT_T, MODE>(ADD ? axpby(g.alpha, p, g.beta, (float)d[q][e])
+                                                        : g.alpha * p);
+        }
+        *reinterpret_cast<o4*>(tile + epi_off<BN>(r, ch0 + q) + 4 * lk) = v;
+      }
+    }
+  }
+  __syncthreads();
+  if (diag_tile) {
+    if (tid < BM) {
+      const int r = tid, c8 = r & ~7;
+      for (int e = 0; e < (r & 7); ++e)
+        tile[epi_off<BN>(r, c8 >> 3) + e] = tile[epi_off<BN>(c8 + e, c8 >> 3) + (r & 7)];
+    }
+    __syncthreads();
+  }
+  const bool vec_rows = (g.ldc % 8 == 0) && (g.sc % 8 == 0) &&
+                        ((reinterpret_cast<uintptr_t>(g.c) | reinterpret_cast<uintptr_t>(g.c_diag)) & 15) == 0;
+  const bool vec_cols = g.ldct % 8 == 0 && g.sct % 8 == 0 && (reinterpret_cast<uintptr_t>(g.ct) & 15) == 0;
+  const int G = lane >> 4, i16 = lane & 15;
+  if (!diag_tile && m0 + BM <= g.m_lim && n0 + BN <= g.n_lim && vec_rows && vec_cols) {
+    // A whole tile: every LDS read of a batch is issued before its first store.
+    constexpr int ROWS = BM * CH / NT, STEP = NT / CH, BATCH = 8;
+    static_assert(ROWS % BATCH == 0, "row batches");
+    const int r0 = tid / CH, ch = tid % CH;
+    if (C || CD) {
+#pragma unroll
+      for (int b = 0; b < ROWS; b += BATCH) {
+        u4 v[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+          v[i] = *reinterpret_cast<const u4*>(tile + epi_off<BN>(r0 + (b + i) * STEP, ch));
+        const int64_t at = (int64_t)(m0 + r0 + b * STEP) * g.ldc + n0 + 8 * ch;
+        if (C) {
+#pragma unroll
+          for (int i = 0; i < BATCH; ++i)
+            *reinterpret_cast<u4*>(C + at + (int64_t)(i * STEP) * g.ldc) = v[i];
+        }
+        if (CD) {
+#pragma unroll
+          for (int i = 0; i < BATCH; ++i)
+            *reinterpret_cast<u4*>(CD + at + (int64_t)(i * STEP) * g.ldc) = v[i];
+        }
+      }
+    }
+    if (CT) {
+      constexpr int ITEMS = (BM / 32) * (BN / 16) / CFG::waves;
+      static_assert(ITEMS % BATCH == 0 && CFG::waves % (BM / 32) == 0, "column batches");
+      constexpr int CSTEP = 16 * CFG::waves / (BM / 32);  // columns between a wave's items
+      const int r8 = 32 * (wave % (BM / 32)) + 8 * G, c0 = 16 * (wave / (BM / 32));
+      const int row = r8 + (i16 >> 2);
+#pragma unroll
+      for (int b = 0; b < ITEMS; b += BATCH) {
+        u4 v[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+          const int ch2 = (c0 + (b + i) * CSTEP) / 8 + ((i16 & 3) >> 1);
+          const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_v4i16_t)(tile + epi_off<BN>(row, ch2) + 4 * (i16 & 1)));
+          const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_v4i16_t)(tile + epi_off<BN>(row + 4, ch2) + 4 * (i16 & 1)));
+          v[i] = __builtin_bit_cast(u4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+        const int64_t col = n0 + c0 + b * CSTEP + i16;
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+          *reinterpret_cast<u4*>(CT + (col + i * CSTEP) * g.ldct + m0 + r8) = v[i];
+        if (g.sym && CD) {
+#pragma unroll
+          for (int i = 0; i < BATCH; ++i)
+            *reinterpret_cast<u4*>(CD + (col + i * CSTEP) * g.ldc + m0 + r8) = v[i];
+        }
+      }
+    }
+    return;
+  }
+  if (C || CD) {
+    for (int q = tid; q < BM * CH; q += NT) {
+      const int r = q / CH, ch = q % CH;
+      const int gr = m0 + r, gc = n0 + 8 * ch;
+      if (gr >= g.m_lim || gc >= g.n_lim || (diag_tile && ch < (r >> 3))) continue;
+      const OUT_T* src = tile + epi_off<BN>(r, ch);
+      if (gc + 8 <= g.n_lim && vec_rows && !(CD && gr >= gc && gr < gc + 8)) {
+        const u4 v = *reinterpret_cast<const u4*>(src);
+        if (C) *reinterpret_cast<u4*>(C + (int64_t)gr * g.ldc + gc) = v;
+        if (CD) *reinterpret_cast<u4*>(CD + (int64_t)gr * g.ldc + gc) = v;
+      } else {
+        for (int e = 0; e < 8; ++e) {
+          const int c = gc + e;
+          if (c >= g.n_lim) continue;
+          if (C) C[(int64_t)gr * g.ldc + c] = src[e];
+          if (CD) CD[(int64_t)gr * g.ldc + c] = (OUT_T)((float)src[e] + (gr == c ? g.diag_shift : 0.f));
+        }
+      }
+    }
+  }
+  if (CT) {
+    for (int it = wave; it < (BM / 32) * (BN / 16); it += CFG::waves) {
+      const int r8 = 32 * (it % (BM / 32)) + 8 * G, cc = it / (BM / 32);
+      const int row = r8 + (i16 >> 2), ch = 2 * cc + ((i16 & 3) >> 1);
+      const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_v4i16_t)(tile + epi_off<BN>(row, ch) + 4 * (i16 & 1)));
+      const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_v4i16_t)(tile + epi_off<BN>(row + 4, ch) + 4 * (i16 & 1)));
+      const int c = 16 * cc + i16;
+      const int gr = m0 + r8, gc = n0 + c;
+      if (gc >= g.n_lim || gr >= g.m_lim || (diag_tile && (r8 >> 3) >= (c >> 3))) continue;
+      OUT_T v[8];
+      __builtin_memcpy(v, &lo, 8);
+      __builtin_memcpy(v + 4, &hi, 8);
+      if (gr + 8 <= g.m_lim && vec_cols) {
+        u4 w;
+        __builtin_memcpy(&w, v, 16);
+        *reinterpret_cast<u4*>(CT + (int64_t)gc * g.ldct + gr) = w;
+        if (g.sym && CD) *reinterpret_cast<u4*>(CD + (int64_t)gc * g.ldc + gr) = w;
+      } else {
+        for (int e = 0; e < 8; ++e) {
+          if (gr + e >= g.m_lim) continue;
+          CT[(int64_t)gc * g.ldct + gr + e] = v[e];
+          if (g.sym && CD) CD[(int64_t)gc * g.ldc + gr + e] = v[e];
+        }
+      }
+    }
+  }
+}
+
+template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
+__device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
+#ifdef __HIP_DEVICE_COMPILE__  // the host pass has no buffer-resource type
+  constexpr int DEPTH = CFG::depth, HM = CFG::HM, HN = CFG::HN, FI = CFG::FI, FJ = CFG::FJ;
+  constexpr int L = CFG::LA, W = CFG::waves;
+  constexpr int BM = CFG::BM, BN = CFG::BN;
+  using V = typename Mfma<T>::vec;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  T* lds_a = reinterpret_cast<T*>(smem);           // [buffer][half][HM][64]
+  T* lds_b = lds_a + 4 * CFG::a_half;              // [buffer][half][HN][64], or [64][HN] (BKN)
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / CFG::WN, wn = wave % CFG::WN;
+  const int tiles = g.sym ? g.tiles_m * (g.tiles_m + 1) / 2 : g.tiles_m * g.tiles_n;
+  const int64_t bidx = w / tiles;
+  const int t = w - (int)bidx * tiles;
+  int tm, tn;
+  if (g.sym) {
+    tri_tile(t, tm, tn);
+  } else {
+    const int group = 8 * g.tiles_n;
+    const int first = (t / group) * 8;
+    const int gm = min(g.tiles_m - first, 8);
+    tm = first + (t % group) % gm;
+    tn = (t % group) / gm;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+  const T* A = reinterpret_cast<const T*>(g.a) + bidx * g.sa + (int64_t)m0 * g.lda;
+  const T* B = reinterpret_cast<const T*>(g.b) + bidx * g.sb + (BKN ? n0 : (int64_t)n0 * g.ldb);
+  // Byte offsets of a lane's 16-byte loads of each half: load j of wave w fills the
+  // 1 KB at 1024 (W j + w) of the half, lane i at +16 i. Rows past the last one
+  // load the last one (outputs that are never stored see them).
+  uint32_t a_off[2][L], b_off[2][L];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+      const int pos = (j * W + wave) * 64 + lane;
+      const int row = pos >> 3, ch = (pos & 7) ^ ((row >> 1) & 7);
+      a_off[h][j] = (uint32_t)min(h * HM + row, g.m - 1 - m0) * (uint32_t)(2 * g.lda) + 16 * ch;
+      if (BKN) {
+        constexpr int NCH = HN / 8;
+        const int krow = pos / NCH;
+        const int c = (pos % NCH) ^ (NCH >= 16 ? 4 * (krow & 3) : 4 * ((krow >> 1) & 1));
+        b_off[h][j] = (uint32_t)krow * (uint32_t)(2 * g.ldb) +
+                      2 * (uint32_t)min(h * HN + c * 8, g.n - 8 - n0);
+      } else {
+        b_off[h][j] = (uint32_t)min(h * HN + row, g.n - 1 - n0) * (uint32_t)(2 * g.ldb) + 16 * ch;
+      }
+    }
+  // Buffer resources from the tile's first row to the operand's end: an address
+  // is a scalar stage offset plus the lane's offset.
+  const uint32_t a_bytes = (uint32_t)(2 * ((g.m - 1 - m0) * g.lda + g.k));
+  const uint32_t b_bytes = (uint32_t)(BKN ? 2 * ((g.k - 1) * g.ldb + g.n - n0)
+                                          : 2 * ((g.n - 1 - n0) * g.ldb + g.k));
+  const auto a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
+  const auto b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, b_bytes, 0x00020000);
+  const int b_step = BKN ? (int)(2 * DEPTH * g.ldb) : 2 * DEPTH;  // bytes per stage
+  const int n_stages = g.k / DEPTH;
+  auto load_a = [&](int kt, int buf, int h) {
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          a_rsrc, (lds_ptr_t)(lds_a + (2 * buf + h) * CFG::a_half + (j * W + wave) * 512), 16,
+          a_off[h][j], kt * (2 * DEPTH), 0, 0);
+  };
+  auto load_b = [&](int kt, int buf, int h) {
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          b_rsrc, (lds_ptr_t)(lds_b + (2 * buf + h) * CFG::b_half + (j * W + wave) * 512), 16,
+          b_off[h][j], kt * b_step, 0, 0);
+  };
+  // The addend's tile, as the epilogue lays it out, goes to the ring's slots once
+  // their last stage has been read: slot s holds tile rows s SLOT_ROWS onwards.
+  constexpr int SLOT_ROWS = CFG::a_half / BN;
+  constexpr int D_SLOTS = BM / SLOT_ROWS;  // 8: every slot; 4: the A slots
+  static_assert(CFG::a_half == CFG::b_half && (D_SLOTS == 8 || D_SLOTS == 4), "slot layout");
+  const T* D = ADD ? reinterpret_cast<const T*>(g.d) + bidx * g.sd + (int64_t)m0 * g.ldd + n0 : nullptr;
+  const uint32_t d_bytes = ADD ? (uint32_t)(2 * ((g.m_lim - 1 - m0) * g.ldd + g.n_lim - n0)) : 0;
+  const auto d_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)D, 0, d_bytes, 0x00020000);
+  auto load_d = [&](int slot) {
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+      const int pos = (j * W + wave) * 64 + lane;
+      const int row = slot * SLOT_ROWS + pos / (BN / 8);
+      const int c = ((pos % (BN / 8)) ^ epi_swz(row)) * 8;
+      const uint32_t off = (uint32_t)min(row, g.m_lim - 1 - m0) * (uint32_t)(2 * g.ldd) +
+                           2 * (uint32_t)min(c, g.n_lim - 8 - n0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          d_rsrc, (lds_ptr_t)(lds_a + slot * CFG::a_half + (j * W + wave) * 512), 16, off, 0, 0, 0);
+    }
+  };
+
+  const int lrow = lane & 31, lk = lane >> 5;
+  const int sw = (lrow >> 1) & 7;
+  const T* a_rd[4];
+  const T* b_rd[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    a_rd[ks] = lds_a + (wm * FI * 32 + lrow) * DEPTH + (((2 * ks + lk) ^ sw) << 3);
+    b_rd[ks] = lds_b + (wn * FJ * 32 + lrow) * DEPTH + (((2 * ks + lk) ^ sw) << 3);
+  }
+  // BKN: chunk ch of k-row r of a half sits at ch ^ (4 (r % 4)) (128 columns) or
+  // ch ^ (4 (r / 2 % 2)) (64 columns).
+  const int G = lane >> 4, i16 = lane & 15;
+  const T* b_kn[FJ];
+#pragma unroll
+  for (int j = 0; j < FJ; ++j) {
+    const int col = (wn * FJ + j) * 32 + 16 * (G & 1) + 4 * (i16 & 3);
+    const int kr = i16 >> 2;  // k-row of the lane, modulo 4
+    const int x = HN >= 128 ? 4 * kr : 4 * (kr >> 1);
+    b_kn[j] = lds_b + (8 * (G >> 1) + kr) * HN + (((col >> 3) ^ x) << 3) + (col & 7);
+  }
+  auto read_a = [&](V (&f)[FI][4], int ks, int buf, int h) {
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+      f[i][ks] = *reinterpret_cast<const V*>(a_rd[ks] + (2 * buf + h) * CFG::a_half + i * 32 * DEPTH);
+  };
+  auto read_b = [&](V (&f)[FJ][4], int ks, int buf, int h) {
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) {
+      if (BKN) {
+        const T* p = b_kn[j] + (2 * buf + h) * CFG::b_half + ks * 16 * HN;
+        v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p));
+        v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p + 4 * HN));
+        f[j][ks] = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      } else {
+        f[j][ks] = *reinterpret_cast<const V*>(b_rd[ks] + (2 * buf + h) * CFG::b_half + j * 32 * DEPTH);
+      }
+    }
+  };
+
+  f32x16 acc[2 * FI][2 * FJ];
+#pragma unroll
+  for (int i = 0; i < 2 * FI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * FJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  const bool diag_tile = g.sym && tm == tn;
+  const bool skip1x = m0 + HM >= g.m_lim, skipx1 = n0 + HN >= g.n_lim;
+  const bool do01 = !skipx1, do11 = !skip1x && !skipx1, do10 = !skip1x && !diag_tile;
+
+  V a[FI][4], bx[FJ][4], by[FJ][4];
+#define QUAD_FENCE __builtin_amdgcn_sched_barrier(0);
+#define QUAD_SYNC(VM)                                                           \
+  QUAD_FENCE                                                                    \
+  wait_vm<VM, 4 * FI>();                                                        \
+  __builtin_amdgcn_s_barrier();                                                 \
+  QUAD_FENCE
+  // One k-step of a quadrant; the MFMA takes B first, so that a lane holds 4
+  // consecutive columns of one row.
+  auto multiply = [&](auto qi_, auto qj_, int ks, V (&b)[FJ][4]) {
+    constexpr int qi = decltype(qi_)::value, qj = decltype(qj_)::value;
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+#pragma unroll
+      for (int j = 0; j < FJ; ++j)
+        acc[qi * FI + i][qj * FJ + j] = Mfma<T>::run(b[j][ks], a[i][ks], acc[qi * FI + i][qj * FJ + j]);
+    QUAD_FENCE
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  // One stage. b0 holds B0(kt) at entry; b1 holds B0(kt + 1) at exit.
+  // tail 0: two more stages follow at least; 1: one; 2: none.
+  auto stage = [&](auto buf_, auto tail_, int kt, V (&b0)[FJ][4], V (&b1)[FJ][4]) {
+    constexpr int buf = decltype(buf_)::value, tail = decltype(tail_)::value;
+    constexpr int dA = ADD ? L : 0, dB = D_SLOTS == 8 ? dA : 0;
+    // rows half 0 x columns half 0; B1(kt) is read
+    QUAD_SYNC((tail != 2 ? 3 * L : dA + 2 * dB))
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      multiply(I0{}, I0{}, ks, b0);
+      read_b(b1, ks, buf, 1);
+      if (ks == 0) {
+        if (tail != 2) load_a(kt + 1, buf ^ 1, 1);
+        else if (dA) load_d(2 * (buf ^ 1) + 1);
+      }
+      QUAD_FENCE
+    }
+    // 0 x 1; A1(kt) replaces A0(kt)
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (do01) multiply(I0{}, I1{}, ks, b1);
+      read_a(a, ks, buf, 1);
+      if (ks == 0) {
+        if (tail == 0) load_b(kt + 2, buf, 0);
+        else if (dB) load_d(4 + 2 * buf);
+      }
+      QUAD_FENCE
+    }
+    // 1 x 1; B0(kt + 1) replaces B1(kt)
+    if (tail != 2 || ADD) {
+      QUAD_SYNC((tail == 0 ? 3 * L : tail == 1 ? 2 * L + dB : 63))
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (do11) multiply(I1{}, I1{}, ks, b1);
+      if (tail != 2) read_b(b1, ks, buf ^ 1, 0);
+      if (ks == 0) {
+        if (tail == 0) load_a(kt + 2, buf, 0);
+        else if (dA) load_d(2 * buf);
+      }
+      QUAD_FENCE
+    }
+    // 1 x 0; A0(kt + 1) replaces A1(kt)
+    if (tail == 2 && ADD) {
+      QUAD_SYNC(63)
+      load_d(2 * buf + 1);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (do10) multiply(I1{}, I0{}, ks, b0);
+      if (tail != 2) read_a(a, ks, buf ^ 1, 0);
+      if (ks == 0) {
+        if (tail == 0) load_b(kt + 2, buf, 1);
+        else if (dB) load_d(5 + 2 * buf);
+      }
+      QUAD_FENCE
+    }
+  };
+  auto first_reads = [&](int buf, V (&b)[FJ][4]) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) read_b(b, ks, buf, 0);
+    QUAD_FENCE
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) read_a(a, ks, buf, 0);
+  };
+
+  // Stage kt sits in buffer (kt + n_stages) & 1, so that the last two stages
+  // always sit in buffers 0 and 1.
+  const int p0 = n_stages & 1;
+  load_b(0, p0, 0);
+  load_a(0, p0, 0);
+  load_b(0, p0, 1);
+  load_a(0, p0, 1);
+  load_b(1, p0 ^ 1, 0);
+  load_a(1, p0 ^ 1, 0);
+  load_b(1, p0 ^ 1, 1);
+  QUAD_SYNC((5 * L))
+  int kt = 0;
+  if (p0) {
+    first_reads(1, by);
+    stage(I1{}, I0{}, 0, by, bx);
+    kt = 1;
+  } else {
+    first_reads(0, bx);
+  }
+  for (; kt < n_stages - 2; kt += 2) {
+    stage(I0{}, I0{}, kt, bx, by);
+    stage(I1{}, I0{}, kt + 1, by, bx);
+  }
+  stage(I0{}, I1{}, n_stages - 2, bx, by);
+  stage(I1{}, I2{}, n_stages - 1, by, bx);
+#undef QUAD_FENCE
+#undef QUAD_SYNC
+  quad_epilogue<T, OUT_T, MODE, CFG, ADD>(g, acc, bidx, m0, n0, wave, lane, skip1x, skipx1, diag_tile,
+                                          smem);
+#endif
 }
 
 // XCD-aware order: the hardware deals workgroup b to XCD b % 8, and an XCD's
@@ -733,6 +1230,13 @@ __global__ __launch_bounds__(CFG::threads, 1) void gemm_nt_pipe_kernel(GemmArgs 
                                                   g.xcd_group));
 }
 
+template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
+__global__ __launch_bounds__(CFG::threads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+gemm_nt_quad_kernel(GemmArgs g, int batch) {
+  quad_tile<T, OUT_T, MODE, CFG, BKN, ADD>(g, xcd_tile((int)blockIdx.x, tile_count(g) * batch,
+                                                       g.xcd_group));
+}
+
 // Several independent products in one launch (the same product of several
 // Newton-Schulz runs): problem q owns workgroups [start[q], start[q + 1]), each
 // range a multiple of 8 long so that every problem keeps its XCD-aware order.
@@ -745,16 +1249,17 @@ struct GemmGroup {
   int count;
 };
 
-template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN>
-__global__ __launch_bounds__(CFG::threads, 1) void gemm_nt_pipe_group_kernel(GemmGroup grp) {
+template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
+__global__ __launch_bounds__(CFG::threads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+gemm_nt_quad_group_kernel(GemmGroup grp) {
   int q = 0;
   for (int j = 1; j < grp.count; ++j)
     if ((int)blockIdx.x >= grp.start[j]) q = j;
-  const GemmArgs& g = grp.g[q];
+  const GemmArgs g = grp.g[q];
   const int w = xcd_tile((int)blockIdx.x - grp.start[q], tile_count(g) * grp.batch[q],
-                        g.xcd_group);
+                         g.xcd_group);
   if (w < 0) return;  // the whole workgroup: w depends on blockIdx only
-  pipe_tile<T, OUT_T, MODE, CFG, BKN>(g, w);
+  quad_tile<T, OUT_T, MODE, CFG, BKN, ADD>(g, w);
 }
 
 // ---- float32 products -----------------------------------------------------------
@@ -982,13 +1487,34 @@ int launch_pipe(const Problem& p, hipStream_t stream) {
   return launch_pipe_kn<T, OUT_T, MODE, CFG, false>(p, stream);
 }
 
-// One launch of up to kMaxGroup products on one tile configuration with
-// 64-deep stages, longest k first (its tiles take longest, so they start first).
-template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN>
-int launch_pipe_group_kn(const std::vector<const Problem*>& ps, hipStream_t stream) {
-  constexpr size_t lds_bytes = pipe_lds_bytes<CFG>();
-  constexpr auto kern = gemm_nt_pipe_group_kernel<T, OUT_T, MODE, CFG, BKN>;
+template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
+int launch_quad_kn(const Problem& p, hipStream_t stream) {
+  constexpr size_t lds_bytes = CFG::lds_bytes;
+  constexpr auto kern = gemm_nt_quad_kernel<T, OUT_T, MODE, CFG, BKN, ADD>;
   DIONW_TRY(allow_lds<kern>(lds_bytes));
+  GemmArgs g;
+  const int64_t wgs = pipe_args<CFG>(p, g);
+  if (wgs < 0) return kInvalid;
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(CFG::threads), lds_bytes, stream, g,
+                     (int)p.batch);
+  return check_launch("gemm_nt_quad");
+}
+
+template <typename T, typename OUT_T, int MODE, typename CFG>
+int launch_quad(const Problem& p, hipStream_t stream) {
+  if (p.g.d)
+    return p.g.b_kn ? launch_quad_kn<T, OUT_T, MODE, CFG, true, true>(p, stream)
+                    : launch_quad_kn<T, OUT_T, MODE, CFG, false, true>(p, stream);
+  return p.g.b_kn ? launch_quad_kn<T, OUT_T, MODE, CFG, true, false>(p, stream)
+                  : launch_quad_kn<T, OUT_T, MODE, CFG, false, false>(p, stream);
+}
+
+// One launch of up to kMaxGroup products on one tile configuration, longest k
+// first (its tiles take longest, so they start first).
+template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
+int launch_quad_group_kn(const std::vector<const Problem*>& ps, hipStream_t stream) {
+  constexpr auto kern = gemm_nt_quad_group_kernel<T, OUT_T, MODE, CFG, BKN, ADD>;
+  DIONW_TRY(allow_lds<kern>(CFG::lds_bytes));
   std::vector<const Problem*> order(ps);
   std::stable_sort(order.begin(), order.end(),
                    [](const Problem* a, const Problem* b) { return a->g.k > b->g.k; });
@@ -1006,24 +1532,27 @@ int launch_pipe_group_kn(const std::vector<const Problem*>& ps, hipStream_t stre
       return kInvalid;
     }
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)start), dim3(CFG::threads), lds_bytes, stream, grp);
-  return check_launch("gemm_nt_pipe_group");
+  hipLaunchKernelGGL(kern, dim3((unsigned)start), dim3(CFG::threads), CFG::lds_bytes, stream, grp);
+  return check_launch("gemm_nt_quad_group");
 }
 
-// Tile of a grouped launch: 256x256 (16 waves, one workgroup per CU) or
-// 128x128 (4 waves, two per CU).
+// Tile of a grouped launch.
 enum GroupTile : int { kNoGroup = 0, kGroupBig = 1, kGroupMid = 2 };
 
+template <typename T, typename OUT_T, int MODE, typename CFG>
+int launch_quad_group(const std::vector<const Problem*>& ps, hipStream_t stream) {
+  const bool kn = ps[0]->g.b_kn, add = ps[0]->g.d != nullptr;
+  if (add)
+    return kn ? launch_quad_group_kn<T, OUT_T, MODE, CFG, true, true>(ps, stream)
+              : launch_quad_group_kn<T, OUT_T, MODE, CFG, false, true>(ps, stream);
+  return kn ? launch_quad_group_kn<T, OUT_T, MODE, CFG, true, false>(ps, stream)
+            : launch_quad_group_kn<T, OUT_T, MODE, CFG, false, false>(ps, stream);
+}
+
 template <typename T, typename OUT_T, int MODE>
-int launch_pipe_group(const std::vector<const Problem*>& ps, GroupTile tile, hipStream_t stream) {
-  using Big64 = PipeCfg<256, 256, 4, 4, 2, 64>;
-  using Mid64 = PipeCfg<128, 128, 2, 2, 2, 64>;
-  const bool kn = ps[0]->g.b_kn;
-  if (tile == kGroupMid)
-    return kn ? launch_pipe_group_kn<T, OUT_T, MODE, Mid64, true>(ps, stream)
-              : launch_pipe_group_kn<T, OUT_T, MODE, Mid64, false>(ps, stream);
-  return kn ? launch_pipe_group_kn<T, OUT_T, MODE, Big64, true>(ps, stream)
-            : launch_pipe_group_kn<T, OUT_T, MODE, Big64, false>(ps, stream);
+int launch_group_typed(const std::vector<const Problem*>& ps, GroupTile tile, hipStream_t stream) {
+  if (tile == kGroupMid) return launch_quad_group<T, OUT_T, MODE, MidTile>(ps, stream);
+  return launch_quad_group<T, OUT_T, MODE, BigTile>(ps, stream);
 }
 
 // Workgroups a tile size yields (symmetric products: upper-triangle tiles).
@@ -1032,56 +1561,50 @@ int64_t wgs_of(const Problem& p, int tile) {
   return p.batch * (p.g.sym ? tm * (tm + 1) / 2 : tm * tn);
 }
 
-// Rounds of workgroups over the 256 CUs (one 256x256 or two 128x128 per CU),
-// in units of one 256x256 round: a 128x128 round counts 2 * 128^2 / 256^2 *
-// 1.3 (the smaller tile's rate is about 1/1.3 of the 256x256 tile's: with 1.2,
-// MoE-Muon's 1408-row symmetric products took the smaller tile and ran 2.4%
-// slower than on 256x256 tiles, while the MoE products that keep it are faster
-// there).
-// Both in twentieths of a 256x256 round (a 128x128 round is 0.65).
-constexpr int kBigRound = 20, kMidRound = 13;
-int64_t big_cost(const Problem& p) { return kBigRound * ((wgs_of(p, 256) + 255) / 256); }
-int64_t mid_cost(const Problem& p) { return kMidRound * ((wgs_of(p, 128) + 511) / 512); }
+// Estimated time of a product on either tile in stage times of a 256x256 tile
+// (64 deep, 1.0 to 1.5 us by clock): rounds of one workgroup per CU, each round
+// its stages plus a fixed part (first loads, epilogue). A 128x128 tile's stage
+// is 0.38 of a 256x256 one's (0.25 of its work), its fixed part 2.6 against 8.
+// Measured, 256x256 / 128x128 tiles, us: 16 x 1024^3 with addend 32 / 35 (160 /
+// 576 tiles), 36 x 768^3 31 / 40, 64 x 1408 x 1408 x 2048 324 / 347, 16 x 1024 x
+// 4096 x 1024 149 / 187; few or ragged tiles: 3584^3 70 / 60, 28 x 576^3 23 /
+// 19, 128 x 384^3 37 / 30, 1024^3 27 / 14.
+double big_cost(const Problem& p) {
+  return (double)((wgs_of(p, 256) + 255) / 256) * (p.g.k / 64.0 + 8.0);
+}
+double mid_cost(const Problem& p) {
+  return (double)((wgs_of(p, 128) + 255) / 256) * (0.38 * p.g.k / 64.0 + 2.6);
+}
+
+// Whether the quadrant tiles take a product: 64-deep stages, two at least; an
+// addend in 16-byte rows; operand extents in 32-bit byte offsets.
+bool quad_ok(const Problem& p) {
+  const GemmArgs& g = p.g;
+  constexpr int64_t kReach = (int64_t)1 << 31;
+  auto reach = [](int64_t rows, int64_t ld) { return 2 * rows * ld < kReach; };
+  return g.k % 64 == 0 && g.k >= 128 && reach(g.m, g.lda) && reach(g.b_kn ? g.k : g.n, g.ldb) &&
+         (!g.d || (g.ldd % 8 == 0 && g.sd % 8 == 0 && g.n_lim % 8 == 0 && aligned16(g.d) &&
+                   reach(g.m_lim, g.ldd)));
+}
 
 template <typename T, typename OUT_T, int MODE>
 int launch_typed(const Problem& p, hipStream_t stream) {
-  auto wgs = [&](int tile) { return wgs_of(p, tile); };
-  // 256x256 tiles run 16 waves of 64x64, 128x128 tiles 4 waves of 64x64. A k
-  // depth that is a multiple of 64 takes 64-deep stages in a two-stage ring (half
-  // the barriers per MFMA of 32-deep stages); other multiples of 32, four
-  // 32-deep stages.
-  using Big64 = PipeCfg<256, 256, 4, 4, 2, 64>;
-  using Mid64 = PipeCfg<128, 128, 2, 2, 2, 64>;
+  // Depths that are an odd multiple of 32 (and what quad_ok refuses) run 32-deep
+  // stages in a ring of four.
   using Big32 = PipeCfg<256, 256, 4, 4, 4, 32>;
   using Mid32 = PipeCfg<128, 128, 2, 2, 4, 32>;
-  const bool k64 = p.g.k % 64 == 0, k32 = p.g.k % 32 == 0;
+  const bool k32 = p.g.k % 32 == 0;
   if (p.g.b_kn && !k32) {
     set_error("gemm: a [k, n] B operand needs k to be a multiple of 32");
     return kInvalid;
   }
-#ifdef DIONW_FORCE_KERNEL
-  // Tuning builds only: one tile shape for every product it can run.
-  if (DIONW_FORCE_KERNEL == 1 && k32) {
-    if (k64) return launch_pipe<T, OUT_T, MODE, Big64>(p, stream);
-    return launch_pipe<T, OUT_T, MODE, Big32>(p, stream);
-  }
-  if (DIONW_FORCE_KERNEL == 2 && k32) {
-    if (k64) return launch_pipe<T, OUT_T, MODE, Mid64>(p, stream);
-    return launch_pipe<T, OUT_T, MODE, Mid32>(p, stream);
-  }
-  if (DIONW_FORCE_KERNEL == 3 && !p.g.b_kn) return launch_cfg<T, OUT_T, 128, 128, 2, 2, MODE>(p, stream);
-  if (DIONW_FORCE_KERNEL == 4 && !p.g.b_kn) return launch_cfg<T, OUT_T, 64, 64, 2, 2, MODE>(p, stream);
-#endif
-  if (k32) {
-    // The smaller tile wins when the big one leaves CUs idle or pads a ragged side.
-    if (big_cost(p) <= mid_cost(p)) {
-      if (k64) return launch_pipe<T, OUT_T, MODE, Big64>(p, stream);
-      return launch_pipe<T, OUT_T, MODE, Big32>(p, stream);
-    }
-    if (k64) return launch_pipe<T, OUT_T, MODE, Mid64>(p, stream);
-    return launch_pipe<T, OUT_T, MODE, Mid32>(p, stream);
-  }
-  if (wgs(128) >= 512) return launch_cfg<T, OUT_T, 128, 128, 2, 2, MODE>(p, stream);
+  if (quad_ok(p))
+    return big_cost(p) <= mid_cost(p) ? launch_quad<T, OUT_T, MODE, BigTile>(p, stream)
+                                      : launch_quad<T, OUT_T, MODE, MidTile>(p, stream);
+  if (k32)
+    return big_cost(p) <= mid_cost(p) ? launch_pipe<T, OUT_T, MODE, Big32>(p, stream)
+                                      : launch_pipe<T, OUT_T, MODE, Mid32>(p, stream);
+  if (wgs_of(p, 128) >= 512) return launch_cfg<T, OUT_T, 128, 128, 2, 2, MODE>(p, stream);
   return launch_cfg<T, OUT_T, 64, 64, 2, 2, MODE>(p, stream);
 }
 
@@ -1121,43 +1644,38 @@ int launch(const Problem& p, hipStream_t stream) {
   return kInvalid;
 }
 
-// Whether one grouped launch beats one launch per product, and on which tile.
-// Time in 256x256 rounds times k (a round of 256x256 tiles over depth k costs
-// k, a round of two 128x128 tiles per CU kGroupMidRate k: the rate the grouping
-// choices were measured with, e.g. gram-ns's lone-run pair on 128x128 tiles,
-// 1.35 -> 1.32 ms; the launcher's own tile rule counts kMidRound / kBigRound).
-// Alone, each product takes its better tile (the launcher's rule); grouped, the
-// tiles of all of them fill the
-// CUs longest first, which costs their total work over the CUs plus about half
-// a round of the shortest tiles, and no less than the longest tile.
-//
-// The same product of several runs (walk_groups' positions) groups on 256x256
-// tiles on that estimate alone. Two independent products of one run, each one
-// round of workgroups or less, also count the ramp and drain of a launch
-// (kRamp, about 11 us: a third of a 256x256 round at k = 1024) and may group on
-// either tile: two launches of one round each cost two ramps; one launch of
-// both, one ramp and the rounds their tiles fill together. (Counting the ramp
-// for the runs' positions too measured slower on GPT-2-small's runs, whose
-// products then group on 128x128 tiles.)
-constexpr double kRamp = 340.0;
-constexpr double kGroupMidRate = 0.6;
+// Whether one grouped launch beats one launch per product, and on which tile, in
+// the units of big_cost. Alone, each product takes its better tile; grouped, the
+// tiles of all of them fill the CUs longest first, which costs the longest tile
+// where they are one round, else their total work over the CUs plus about half a
+// round of the shortest tiles. A launch of one round or less, and each of two
+// independent products of one run (pair), also costs its ramp and drain (kRamp,
+// about 6 us).
+constexpr double kRamp = 5.3;
 
 GroupTile group_plan(const std::vector<const Problem*>& ps, bool pair) {
-  const double ramp = pair ? kRamp : 0.0;
-  double separate = 0.0, big = 0.0, mid = 0.0, kmax = 0.0, kmin = 1e300;
+  double separate = 0.0, ramp = 0.0, work[2] = {}, longest[2] = {}, shortest[2] = {1e300, 1e300};
+  int64_t wgs[2] = {};
   for (const Problem* p : ps) {
-    const double k = (double)p->g.k;
-    separate += ramp + k * (double)std::min(big_cost(*p), mid_cost(*p)) / kBigRound;
-    big += k * (double)wgs_of(*p, 256) / 256.0;
-    mid += kGroupMidRate * k * (double)wgs_of(*p, 128) / 512.0;
-    kmax = std::max(kmax, k);
-    kmin = std::min(kmin, k);
+    const double k = p->g.k / 64.0, tile[2] = {k + 8.0, 0.38 * k + 2.6};
+    const double alone[2] = {big_cost(*p), mid_cost(*p)};
+    const int best = alone[0] <= alone[1] ? 0 : 1;
+    const bool ramps = pair || wgs_of(*p, best ? 128 : 256) <= 256;
+    if (ramps) ramp = kRamp;
+    separate += (ramps ? kRamp : 0.0) + alone[best];
+    for (int c = 0; c < 2; ++c) {
+      const int64_t n = wgs_of(*p, c ? 128 : 256);
+      wgs[c] += n;
+      work[c] += tile[c] * (double)n / 256.0;
+      longest[c] = std::max(longest[c], tile[c]);
+      shortest[c] = std::min(shortest[c], tile[c]);
+    }
   }
-  const double big_total = ramp + std::max(big + 0.5 * kmin, kmax);
-  const double mid_total =
-      pair ? ramp + std::max(mid + 0.5 * kGroupMidRate * kmin, kGroupMidRate * kmax) : 1e300;
-  if (std::min(big_total, mid_total) >= separate) return kNoGroup;
-  return mid_total < big_total ? kGroupMid : kGroupBig;
+  double total[2];
+  for (int c = 0; c < 2; ++c)
+    total[c] = ramp + (wgs[c] <= 256 ? longest[c] : std::max(longest[c], work[c] + 0.5 * shortest[c]));
+  if (std::min(total[0], total[1]) >= separate) return kNoGroup;
+  return total[1] < total[0] ? kGroupMid : kGroupBig;
 }
 
 // Independent products in as few launches as possible: one grouped launch when
@@ -1175,8 +1693,9 @@ GroupTile groups(const std::vector<const Problem*>& live, bool pair = false) {
   bool together = live.size() >= 2 && live.size() <= (size_t)kMaxGroup;
   for (const Problem* p : live)
     together = together && p->elem == live[0]->elem && p->out_mode == live[0]->out_mode &&
-               p->g.b_kn == live[0]->g.b_kn && p->g.k % 64 == 0 && p->batch <= INT32_MAX &&
-               operands_ok(p->g) && !(p->g.b_kn && (p->g.n % 8 || p->g.sym));
+               p->g.b_kn == live[0]->g.b_kn && !p->g.d == !live[0]->g.d && quad_ok(*p) &&
+               p->batch <= INT32_MAX && operands_ok(p->g) &&
+               !(p->g.b_kn && (p->g.n % 8 || p->g.sym));
   return together ? group_plan(live, pair) : kNoGroup;
 }
 
@@ -1189,12 +1708,12 @@ int launch_group(const std::vector<const Problem*>& ps, hipStream_t stream, bool
   }
   if (live[0]->elem == kF16) {
     if (live[0]->out_mode == kOutBf16ViaF16)
-      return launch_pipe_group<_Float16, __bf16, kOutBf16ViaF16>(live, tile, stream);
-    return launch_pipe_group<_Float16, _Float16, kOutSame>(live, tile, stream);
+      return launch_group_typed<_Float16, __bf16, kOutBf16ViaF16>(live, tile, stream);
+    return launch_group_typed<_Float16, _Float16, kOutSame>(live, tile, stream);
   }
   if (live[0]->out_mode == kOutRoundAcc)
-    return launch_pipe_group<__bf16, __bf16, kOutRoundAcc>(live, tile, stream);
-  return launch_pipe_group<__bf16, __bf16, kOutSame>(live, tile, stream);
+    return launch_group_typed<__bf16, __bf16, kOutRoundAcc>(live, tile, stream);
+  return launch_group_typed<__bf16, __bf16, kOutSame>(live, tile, stream);
 }
 
 // ---- Newton-Schulz drivers ---------------------------------------------------
