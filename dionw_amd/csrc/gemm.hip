@@ -749,7 +749,7 @@ struct QuadCfg {
   static constexpr int WM = WM_, WN = WN_, FI = FI_, FJ = FJ_;
   static constexpr int waves = WM * WN, threads = waves * 64;
   static constexpr int HM = WM * FI * 32, HN = WN * FJ * 32;  // half tile rows / columns
-  static constexpr int BM = 2 * HM, BN = 2 * HN;
+  static constexpr int halves = 2, BM = halves * HM, BN = halves * HN;
   static constexpr int depth = 64;
   static constexpr int a_half = HM * depth, b_half = HN * depth;   // elements of a half stage
   static constexpr int LA = a_half / 8 / threads, LB = b_half / 8 / threads;  // loads per lane
@@ -763,12 +763,16 @@ using MidTile = QuadCfg<2, 2, 1, 1>;  // 128x128, 4 waves, two workgroups per CU
 
 // The output tile in LDS: rows of BN elements, 16-byte chunk ch of row r at
 // ch ^ epi_swz(r).
-__device__ __forceinline__ int epi_swz(int r) { return ((r & 3) << 1) | ((r >> 2) & 1) | (r & 8); }
 template <int BN>
-__device__ __forceinline__ int epi_off(int r, int ch) { return r * BN + ((ch ^ epi_swz(r)) << 3); }
+__device__ __forceinline__ int epi_swz(int r) {
+  if (BN >= 128) return ((r & 3) << 1) | ((r >> 2) & 1) | (r & 8);
+  return (r & 2) | ((r >> 2) & 1) | ((r >> 1) & 4);  // two rows of 64 span the banks
+}
+template <int BN>
+__device__ __forceinline__ int epi_off(int r, int ch) { return r * BN + ((ch ^ epi_swz<BN>(r)) << 3); }
 
 template <typename T, typename OUT_T, int MODE, typename CFG, bool ADD>
-__device__ __forceinline__ void quad_epilogue(const GemmArgs& g, f32x16 (&acc)[2 * CFG::FI][2 * CFG::FJ],
+__device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x16 (&acc)[CFG::halves * CFG::FI][CFG::halves * CFG::FJ],
                                               int64_t bidx, int m0, int n0, int wave, int lane,
                                               bool skip1x, bool skipx1, bool diag_tile,
                                               unsigned char* smem) {
@@ -786,10 +790,10 @@ __device__ __forceinline__ void quad_epilogue(const GemmArgs& g, f32x16 (&acc)[2
   __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt(0) lgkmcnt(0): the addend has landed
   __builtin_amdgcn_s_barrier();
 #pragma unroll
-  for (int i = 0; i < 2 * CFG::FI; ++i) {
+  for (int i = 0; i < CFG::halves * CFG::FI; ++i) {
     if (i >= CFG::FI && skip1x) continue;
 #pragma unroll
-    for (int j = 0; j < 2 * CFG::FJ; ++j) {
+    for (int j = 0; j < CFG::halves * CFG::FJ; ++j) {
       if (j >= CFG::FJ && skipx1) continue;
       if (i >= CFG::FI && j < CFG::FJ && diag_tile) continue;
       const int r = (i / CFG::FI) * CFG::HM + (wm * CFG::FI + i % CFG::FI) * 32 + lrow;
@@ -827,9 +831,11 @@ __device__ __forceinline__ void quad_epilogue(const GemmArgs& g, f32x16 (&acc)[2
                         ((reinterpret_cast<uintptr_t>(g.c) | reinterpret_cast<uintptr_t>(g.c_diag)) & 15) == 0;
   const bool vec_cols = g.ldct % 8 == 0 && g.sct % 8 == 0 && (reinterpret_cast<uintptr_t>(g.ct) & 15) == 0;
   const int G = lane >> 4, i16 = lane & 15;
-  if (!diag_tile && m0 + BM <= g.m_lim && n0 + BN <= g.n_lim && vec_rows && vec_cols) {
-    // A whole tile: every LDS read of a batch is issued before its first store.
-    constexpr int ROWS = BM * CH / NT, STEP = NT / CH, BATCH = 8;
+  if (m0 + BM <= g.m_lim && n0 + BN <= g.n_lim && vec_rows && vec_cols) {
+    // A whole tile: every LDS read of a batch is issued before its first store. A
+    // diagonal tile stores its 8x8 blocks on and above the diagonal as they lie and
+    // those above it mirrored.
+    constexpr int ROWS = BM * CH / NT, STEP = NT / CH, BATCH = ROWS < 8 ? ROWS : 8;
     static_assert(ROWS % BATCH == 0, "row batches");
     const int r0 = tid / CH, ch = tid % CH;
     if (C || CD) {
@@ -840,15 +846,22 @@ __device__ __forceinline__ void quad_epilogue(const GemmArgs& g, f32x16 (&acc)[2
         for (int i = 0; i < BATCH; ++i)
           v[i] = *reinterpret_cast<const u4*>(tile + epi_off<BN>(r0 + (b + i) * STEP, ch));
         const int64_t at = (int64_t)(m0 + r0 + b * STEP) * g.ldc + n0 + 8 * ch;
-        if (C) {
 #pragma unroll
-          for (int i = 0; i < BATCH; ++i)
-            *reinterpret_cast<u4*>(C + at + (int64_t)(i * STEP) * g.ldc) = v[i];
-        }
-        if (CD) {
+        for (int i = 0; i < BATCH; ++i) {
+          if (diag_tile && ch < ((r0 + (b + i) * STEP) >> 3)) continue;
+          if (C) *reinterpret_cast<u4*>(C + at + (int64_t)(i * STEP) * g.ldc) = v[i];
+          if (CD) {
+            const int r = r0 + (b + i) * STEP;
+            if (diag_tile && ch == (r >> 3)) {
+              OUT_T x[8];
+              __builtin_memcpy(x, &v[i], 16);
 #pragma unroll
-          for (int i = 0; i < BATCH; ++i)
+              for (int e = 0; e < 8; ++e)
+                if (e == (r & 7)) x[e] = (OUT_T)((float)x[e] + g.diag_shift);
+              __builtin_memcpy(&v[i], x, 16);
+            }
             *reinterpret_cast<u4*>(CD + at + (int64_t)(i * STEP) * g.ldc) = v[i];
+          }
         }
       }
     }
@@ -870,14 +883,13 @@ __device__ __forceinline__ void quad_epilogue(const GemmArgs& g, f32x16 (&acc)[2
               (lds_v4i16_t)(tile + epi_off<BN>(row + 4, ch2) + 4 * (i16 & 1)));
           v[i] = __builtin_bit_cast(u4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         }
-        const int64_t col = n0 + c0 + b * CSTEP + i16;
+        const int c = c0 + b * CSTEP + i16;
 #pragma unroll
-        for (int i = 0; i < BATCH; ++i)
-          *reinterpret_cast<u4*>(CT + (col + i * CSTEP) * g.ldct + m0 + r8) = v[i];
-        if (g.sym && CD) {
-#pragma unroll
-          for (int i = 0; i < BATCH; ++i)
-            *reinterpret_cast<u4*>(CD + (col + i * CSTEP) * g.ldc + m0 + r8) = v[i];
+        for (int i = 0; i < BATCH; ++i) {
+          if (diag_tile && r8 >= ((c + i * CSTEP) & ~7)) continue;
+          *reinterpret_cast<u4*>(CT + (int64_t)(n0 + c + i * CSTEP) * g.ldct + m0 + r8) = v[i];
+          if (g.sym && CD)
+            *reinterpret_cast<u4*>(CD + (int64_t)(n0 + c + i * CSTEP) * g.ldc + m0 + r8) = v[i];
         }
       }
     }
@@ -1020,7 +1032,7 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
     for (int j = 0; j < L; ++j) {
       const int pos = (j * W + wave) * 64 + lane;
       const int row = slot * SLOT_ROWS + pos / (BN / 8);
-      const int c = ((pos % (BN / 8)) ^ epi_swz(row)) * 8;
+      const int c = ((pos % (BN / 8)) ^ epi_swz<BN>(row)) * 8;
       const uint32_t off = (uint32_t)min(row, g.m_lim - 1 - m0) * (uint32_t)(2 * g.ldd) +
                            2 * (uint32_t)min(c, g.n_lim - 8 - n0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -1193,8 +1205,184 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
   stage(I1{}, I2{}, n_stages - 1, by, bx);
 #undef QUAD_FENCE
 #undef QUAD_SYNC
-  quad_epilogue<T, OUT_T, MODE, CFG, ADD>(g, acc, bidx, m0, n0, wave, lane, skip1x, skipx1, diag_tile,
+  tile_epilogue<T, OUT_T, MODE, CFG, ADD>(g, acc, bidx, m0, n0, wave, lane, skip1x, skipx1, diag_tile,
                                           smem);
+#endif
+}
+
+// ---- 64x64 tiles -------------------------------------------------------------------
+//
+// For products of so few tiles that their time is one tile's chain of stages and the
+// launch: 4 waves of one 32x32 fragment each, and a ring of 8 stages (64 deep) per
+// workgroup, so that 7 stages are on their way from the first moment and a stage has
+// six others' time to land. A stage's fragments are read under the MFMAs of the stage
+// before; one barrier per stage. Measured in a chain of launches, us, against 128x128
+// tiles: 1024^3 symmetric with addend 12.1 / 8.7, 512^3 9.1 / 6.6, 256^3 7.4 / 5.9
+// (an empty kernel takes 4.7); a 1 x 1024x1024 Newton-Schulz call 249 / 147.
+struct SmallTile {
+  static constexpr int WM = 2, WN = 2, FI = 1, FJ = 1, waves = 4, threads = 256;
+  static constexpr int BM = 64, BN = 64, depth = 64;
+  [[maybe_unused]] static constexpr int HM = 64, HN = 64, halves = 1;
+  static constexpr int stages = 8, operand = 64 * depth;  // ring depth, elements of an operand's stage
+  static constexpr size_t ring_bytes = (size_t)stages * 2 * operand * 2;
+  static constexpr size_t lds_bytes = ring_bytes + (size_t)BM * BN * 2;
+};
+
+// s_waitcnt for at most 4 n loads in flight, n <= 6.
+__device__ __forceinline__ void wait_small(int n) {
+  switch (n) {
+    case 0: wait_vm<0, 15>(); break;
+    case 1: wait_vm<4, 15>(); break;
+    case 2: wait_vm<8, 15>(); break;
+    case 3: wait_vm<12, 15>(); break;
+    case 4: wait_vm<16, 15>(); break;
+    case 5: wait_vm<20, 15>(); break;
+    default: wait_vm<24, 15>(); break;
+  }
+}
+
+template <typename T, typename OUT_T, int MODE, bool BKN, bool ADD>
+__device__ __forceinline__ void small_tile(const GemmArgs& g, int w) {
+#ifdef __HIP_DEVICE_COMPILE__
+  using CFG = SmallTile;
+  constexpr int DEPTH = CFG::depth, S = CFG::stages, BM = CFG::BM, BN = CFG::BN;
+  using V = typename Mfma<T>::vec;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  T* lds = reinterpret_cast<T*>(smem);  // [stage][A 64x64, B 64x64], then the output tile
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int tiles = g.sym ? g.tiles_m * (g.tiles_m + 1) / 2 : g.tiles_m * g.tiles_n;
+  const int64_t bidx = w / tiles;
+  const int t = w - (int)bidx * tiles;
+  int tm, tn;
+  if (g.sym) {
+    tri_tile(t, tm, tn);
+  } else {
+    const int group = 8 * g.tiles_n;
+    const int first = (t / group) * 8;
+    const int gm = min(g.tiles_m - first, 8);
+    tm = first + (t % group) % gm;
+    tn = (t % group) / gm;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+  const T* A = reinterpret_cast<const T*>(g.a) + bidx * g.sa + (int64_t)m0 * g.lda;
+  const T* B = reinterpret_cast<const T*>(g.b) + bidx * g.sb + (BKN ? n0 : (int64_t)n0 * g.ldb);
+  uint32_t a_off[2], b_off[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int pos = (j * 4 + wave) * 64 + lane;
+    const int row = pos >> 3, ch = (pos & 7) ^ ((row >> 1) & 7);
+    a_off[j] = (uint32_t)min(row, g.m - 1 - m0) * (uint32_t)(2 * g.lda) + 16 * ch;
+    if (BKN) {
+      const int c = (pos & 7) ^ (4 * ((row >> 1) & 1));  // row: the k-row
+      b_off[j] = (uint32_t)row * (uint32_t)(2 * g.ldb) + 2 * (uint32_t)min(c * 8, g.n - 8 - n0);
+    } else {
+      b_off[j] = (uint32_t)min(row, g.n - 1 - n0) * (uint32_t)(2 * g.ldb) + 16 * ch;
+    }
+  }
+  const uint32_t a_bytes = (uint32_t)(2 * ((g.m - 1 - m0) * g.lda + g.k));
+  const uint32_t b_bytes = (uint32_t)(BKN ? 2 * ((g.k - 1) * g.ldb + g.n - n0)
+                                          : 2 * ((g.n - 1 - n0) * g.ldb + g.k));
+  const auto a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
+  const auto b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, b_bytes, 0x00020000);
+  const int b_step = BKN ? (int)(2 * DEPTH * g.ldb) : 2 * DEPTH;
+  const int n_stages = g.k / DEPTH;
+  auto issue = [&](int kt) {
+    T* stage = lds + (kt % S) * (2 * CFG::operand);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr_t)(stage + (j * 4 + wave) * 512), 16,
+                                               a_off[j], kt * (2 * DEPTH), 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          b_rsrc, (lds_ptr_t)(stage + CFG::operand + (j * 4 + wave) * 512), 16, b_off[j],
+          kt * b_step, 0, 0);
+    }
+  };
+  unsigned char* tile = smem + CFG::ring_bytes;
+  if (ADD) {
+    const T* D = reinterpret_cast<const T*>(g.d) + bidx * g.sd + (int64_t)m0 * g.ldd + n0;
+    const uint32_t d_bytes = (uint32_t)(2 * ((g.m_lim - 1 - m0) * g.ldd + g.n_lim - n0));
+    const auto d_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)D, 0, d_bytes, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int pos = (j * 4 + wave) * 64 + lane, row = pos >> 3;
+      const int c = ((pos & 7) ^ epi_swz<BN>(row)) * 8;
+      const uint32_t off = (uint32_t)min(row, g.m_lim - 1 - m0) * (uint32_t)(2 * g.ldd) +
+                           2 * (uint32_t)min(c, g.n_lim - 8 - n0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          d_rsrc, (lds_ptr_t)(reinterpret_cast<T*>(tile) + (j * 4 + wave) * 512), 16, off, 0, 0, 0);
+    }
+  }
+
+  const int lrow = lane & 31, lk = lane >> 5, sw = (lrow >> 1) & 7;
+  int a_rd[4], b_rd[4];  // element offsets in a stage, per k-step
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    a_rd[ks] = (wm * 32 + lrow) * DEPTH + (((2 * ks + lk) ^ sw) << 3);
+    b_rd[ks] = CFG::operand + (wn * 32 + lrow) * DEPTH + (((2 * ks + lk) ^ sw) << 3);
+  }
+  const int G = lane >> 4, i16 = lane & 15, kr = i16 >> 2;
+  const int kn_col = wn * 32 + 16 * (G & 1) + 4 * (i16 & 3);
+  const int b_kn = CFG::operand + (8 * (G >> 1) + kr) * BN +
+                   (((kn_col >> 3) ^ (4 * (kr >> 1))) << 3) + (kn_col & 7);
+  struct Frags {
+    V a[4], b[4];
+  };
+  auto read = [&](Frags& f, int kt) {
+    const T* stage = lds + (kt % S) * (2 * CFG::operand);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      f.a[ks] = *reinterpret_cast<const V*>(stage + a_rd[ks]);
+      if (BKN) {
+        const T* p = stage + b_kn + ks * 16 * BN;
+        v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p));
+        v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p + 4 * BN));
+        f.b[ks] = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      } else {
+        f.b[ks] = *reinterpret_cast<const V*>(stage + b_rd[ks]);
+      }
+    }
+  };
+  f32x16 acc[1][1];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[0][0][e] = 0.f;
+  // Stage kt is multiplied while stage kt + 1 is read and stage kt - 1 + S requested
+  // (into the slot of kt - 1, which every wave has multiplied).
+  auto step = [&](auto more_, int kt, Frags& now, Frags& next) {
+    if (decltype(more_)::value) {
+      __builtin_amdgcn_sched_barrier(0);
+      wait_small(min(S - 3, n_stages - 2 - kt));
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      read(next, kt + 1);
+      if (kt - 1 + S < n_stages) issue(kt - 1 + S);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) acc[0][0] = Mfma<T>::run(now.b[ks], now.a[ks], acc[0][0]);
+  };
+#pragma unroll 1
+  for (int s = 0; s < min(S - 1, n_stages); ++s) issue(s);
+  wait_small(min(S - 2, n_stages - 1));
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  Frags x, y;
+  read(x, 0);
+  int kt = 0;
+  for (; kt + 2 < n_stages; kt += 2) {
+    step(std::true_type{}, kt, x, y);
+    step(std::true_type{}, kt + 1, y, x);
+  }
+  if (kt + 1 < n_stages) {
+    step(std::true_type{}, kt, x, y);
+    step(std::false_type{}, kt + 1, y, x);
+  } else {
+    step(std::false_type{}, kt, x, y);
+  }
+  tile_epilogue<T, OUT_T, MODE, CFG, ADD>(g, acc, bidx, m0, n0, wave, lane, false, false,
+                                          g.sym && tm == tn, tile);
 #endif
 }
 
@@ -1231,10 +1419,18 @@ __global__ __launch_bounds__(CFG::threads, 1) void gemm_nt_pipe_kernel(GemmArgs 
 }
 
 template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
+__device__ __forceinline__ void product_tile(const GemmArgs& g, int w) {
+  if constexpr (std::is_same<CFG, SmallTile>::value)
+    small_tile<T, OUT_T, MODE, BKN, ADD>(g, w);
+  else
+    quad_tile<T, OUT_T, MODE, CFG, BKN, ADD>(g, w);
+}
+
+template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
 __global__ __launch_bounds__(CFG::threads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-gemm_nt_quad_kernel(GemmArgs g, int batch) {
-  quad_tile<T, OUT_T, MODE, CFG, BKN, ADD>(g, xcd_tile((int)blockIdx.x, tile_count(g) * batch,
-                                                       g.xcd_group));
+gemm_nt_tile_kernel(GemmArgs g, int batch) {
+  product_tile<T, OUT_T, MODE, CFG, BKN, ADD>(g, xcd_tile((int)blockIdx.x, tile_count(g) * batch,
+                                                          g.xcd_group));
 }
 
 // Several independent products in one launch (the same product of several
@@ -1251,7 +1447,7 @@ struct GemmGroup {
 
 template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
 __global__ __launch_bounds__(CFG::threads, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-gemm_nt_quad_group_kernel(GemmGroup grp) {
+gemm_nt_tile_group_kernel(GemmGroup grp) {
   int q = 0;
   for (int j = 1; j < grp.count; ++j)
     if ((int)blockIdx.x >= grp.start[j]) q = j;
@@ -1259,7 +1455,7 @@ gemm_nt_quad_group_kernel(GemmGroup grp) {
   const int w = xcd_tile((int)blockIdx.x - grp.start[q], tile_count(g) * grp.batch[q],
                          g.xcd_group);
   if (w < 0) return;  // the whole workgroup: w depends on blockIdx only
-  quad_tile<T, OUT_T, MODE, CFG, BKN, ADD>(g, w);
+  product_tile<T, OUT_T, MODE, CFG, BKN, ADD>(g, w);
 }
 
 // ---- float32 products -----------------------------------------------------------
@@ -1488,32 +1684,84 @@ int launch_pipe(const Problem& p, hipStream_t stream) {
 }
 
 template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
-int launch_quad_kn(const Problem& p, hipStream_t stream) {
+int launch_tile_kn(const Problem& p, hipStream_t stream) {
   constexpr size_t lds_bytes = CFG::lds_bytes;
-  constexpr auto kern = gemm_nt_quad_kernel<T, OUT_T, MODE, CFG, BKN, ADD>;
+  constexpr auto kern = gemm_nt_tile_kernel<T, OUT_T, MODE, CFG, BKN, ADD>;
   DIONW_TRY(allow_lds<kern>(lds_bytes));
   GemmArgs g;
   const int64_t wgs = pipe_args<CFG>(p, g);
   if (wgs < 0) return kInvalid;
   hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(CFG::threads), lds_bytes, stream, g,
                      (int)p.batch);
-  return check_launch("gemm_nt_quad");
+  return check_launch("gemm_nt_tile");
 }
 
 template <typename T, typename OUT_T, int MODE, typename CFG>
-int launch_quad(const Problem& p, hipStream_t stream) {
+int launch_tile(const Problem& p, hipStream_t stream) {
   if (p.g.d)
-    return p.g.b_kn ? launch_quad_kn<T, OUT_T, MODE, CFG, true, true>(p, stream)
-                    : launch_quad_kn<T, OUT_T, MODE, CFG, false, true>(p, stream);
-  return p.g.b_kn ? launch_quad_kn<T, OUT_T, MODE, CFG, true, false>(p, stream)
-                  : launch_quad_kn<T, OUT_T, MODE, CFG, false, false>(p, stream);
+    return p.g.b_kn ? launch_tile_kn<T, OUT_T, MODE, CFG, true, true>(p, stream)
+                    : launch_tile_kn<T, OUT_T, MODE, CFG, false, true>(p, stream);
+  return p.g.b_kn ? launch_tile_kn<T, OUT_T, MODE, CFG, true, false>(p, stream)
+                  : launch_tile_kn<T, OUT_T, MODE, CFG, false, false>(p, stream);
+}
+
+// Workgroups a tile size yields (symmetric products: upper-triangle tiles).
+int64_t wgs_of(const Problem& p, int tile) {
+  const int64_t tm = (p.g.m + tile - 1) / tile, tn = (p.g.n + tile - 1) / tile;
+  return p.batch * (p.g.sym ? tm * (tm + 1) / 2 : tm * tn);
+}
+
+// The tiles of the 64-deep kernels.
+enum Tile : int { kBig = 0, kMid = 1, kSmall = 2 };
+constexpr int kTileSide[3] = {256, 128, 64};
+
+// Estimated time of one tile of depth k in stage times of a 256x256 tile (64 deep,
+// 1.0 to 1.5 us by clock), with a workgroup on every CU: its stages plus a fixed
+// part (first loads, epilogue).
+double tile_time(int tile, int64_t k) {
+  constexpr double stage[3] = {1.0, 0.38, 0.23}, fixed[3] = {8.0, 2.6, 0.6};
+  return stage[tile] * (double)k / 64.0 + fixed[tile];
+}
+
+// Whether a tile may run `wgs` workgroups: 64x64 tiles only where one round holds
+// them all. Their ring fills a CU's LDS, so that a second round waits for the
+// first, and they read four times the operand bytes of 256x256 ones.
+bool tile_fits(int tile, int64_t wgs) { return tile != kSmall || wgs <= 256; }
+
+// A product's time on a tile: rounds of one workgroup per CU. Measured on 256x256 /
+// 128x128 / 64x64 tiles, us per launch of a chain: 16 x 1024^3 symmetric with addend
+// 32 / 35 / -, 36 x 768^3 31 / 40 / -, 64 x 1408 x 1408 x 2048 324 / 347 / -,
+// 16 x 1024 x 4096 x 1024 149 / 187 / -; 3584^3 69 / 59 / 128, 28 x 576^3 23 / 17 /
+// 29, 128 x 384^3 36 / 28 / 51, 4 x 1024^3 27 / 15 / 22; 1024^3 26 / 14 / 9,
+// 12 x 384^3 18 / 10 / 7, 256^3 16 / 9 / 6 (64 x 64 x 64: 6; an empty kernel: 4.7).
+double product_time(const Problem& p, int tile) {
+  const int64_t wgs = wgs_of(p, kTileSide[tile]);
+  if (!tile_fits(tile, wgs)) return 1e300;
+  return (double)((wgs + 255) / 256) * tile_time(tile, p.g.k);
+}
+int best_tile(const Problem& p) {
+  int best = kBig;
+  for (int c = kMid; c <= kSmall; ++c)
+    if (product_time(p, c) < product_time(p, best)) best = c;
+  return best;
+}
+
+// Whether the 64-deep tiles take a product: an addend in 16-byte rows, operand
+// extents in 32-bit byte offsets, two stages at least (64x64 tiles: one).
+bool tiles_ok(const Problem& p) {
+  const GemmArgs& g = p.g;
+  constexpr int64_t kReach = (int64_t)1 << 31;
+  auto reach = [](int64_t rows, int64_t ld) { return 2 * rows * ld < kReach; };
+  return g.k % 64 == 0 && (g.k >= 128 || best_tile(p) == kSmall) && reach(g.m, g.lda) && reach(g.b_kn ? g.k : g.n, g.ldb) &&
+         (!g.d || (g.ldd % 8 == 0 && g.sd % 8 == 0 && g.n_lim % 8 == 0 && aligned16(g.d) &&
+                   reach(g.m_lim, g.ldd)));
 }
 
 // One launch of up to kMaxGroup products on one tile configuration, longest k
 // first (its tiles take longest, so they start first).
 template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
-int launch_quad_group_kn(const std::vector<const Problem*>& ps, hipStream_t stream) {
-  constexpr auto kern = gemm_nt_quad_group_kernel<T, OUT_T, MODE, CFG, BKN, ADD>;
+int launch_tile_group_kn(const std::vector<const Problem*>& ps, hipStream_t stream) {
+  constexpr auto kern = gemm_nt_tile_group_kernel<T, OUT_T, MODE, CFG, BKN, ADD>;
   DIONW_TRY(allow_lds<kern>(CFG::lds_bytes));
   std::vector<const Problem*> order(ps);
   std::stable_sort(order.begin(), order.end(),
@@ -1533,63 +1781,31 @@ int launch_quad_group_kn(const std::vector<const Problem*>& ps, hipStream_t stre
     }
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)start), dim3(CFG::threads), CFG::lds_bytes, stream, grp);
-  return check_launch("gemm_nt_quad_group");
+  return check_launch("gemm_nt_tile_group");
 }
 
-// Tile of a grouped launch.
-enum GroupTile : int { kNoGroup = 0, kGroupBig = 1, kGroupMid = 2 };
-
 template <typename T, typename OUT_T, int MODE, typename CFG>
-int launch_quad_group(const std::vector<const Problem*>& ps, hipStream_t stream) {
+int launch_tile_group(const std::vector<const Problem*>& ps, hipStream_t stream) {
   const bool kn = ps[0]->g.b_kn, add = ps[0]->g.d != nullptr;
   if (add)
-    return kn ? launch_quad_group_kn<T, OUT_T, MODE, CFG, true, true>(ps, stream)
-              : launch_quad_group_kn<T, OUT_T, MODE, CFG, false, true>(ps, stream);
-  return kn ? launch_quad_group_kn<T, OUT_T, MODE, CFG, true, false>(ps, stream)
-            : launch_quad_group_kn<T, OUT_T, MODE, CFG, false, false>(ps, stream);
+    return kn ? launch_tile_group_kn<T, OUT_T, MODE, CFG, true, true>(ps, stream)
+              : launch_tile_group_kn<T, OUT_T, MODE, CFG, false, true>(ps, stream);
+  return kn ? launch_tile_group_kn<T, OUT_T, MODE, CFG, true, false>(ps, stream)
+            : launch_tile_group_kn<T, OUT_T, MODE, CFG, false, false>(ps, stream);
 }
 
 template <typename T, typename OUT_T, int MODE>
-int launch_group_typed(const std::vector<const Problem*>& ps, GroupTile tile, hipStream_t stream) {
-  if (tile == kGroupMid) return launch_quad_group<T, OUT_T, MODE, MidTile>(ps, stream);
-  return launch_quad_group<T, OUT_T, MODE, BigTile>(ps, stream);
-}
-
-// Workgroups a tile size yields (symmetric products: upper-triangle tiles).
-int64_t wgs_of(const Problem& p, int tile) {
-  const int64_t tm = (p.g.m + tile - 1) / tile, tn = (p.g.n + tile - 1) / tile;
-  return p.batch * (p.g.sym ? tm * (tm + 1) / 2 : tm * tn);
-}
-
-// Estimated time of a product on either tile in stage times of a 256x256 tile
-// (64 deep, 1.0 to 1.5 us by clock): rounds of one workgroup per CU, each round
-// its stages plus a fixed part (first loads, epilogue). A 128x128 tile's stage
-// is 0.38 of a 256x256 one's (0.25 of its work), its fixed part 2.6 against 8.
-// Measured, 256x256 / 128x128 tiles, us: 16 x 1024^3 with addend 32 / 35 (160 /
-// 576 tiles), 36 x 768^3 31 / 40, 64 x 1408 x 1408 x 2048 324 / 347, 16 x 1024 x
-// 4096 x 1024 149 / 187; few or ragged tiles: 3584^3 70 / 60, 28 x 576^3 23 /
-// 19, 128 x 384^3 37 / 30, 1024^3 27 / 14.
-double big_cost(const Problem& p) {
-  return (double)((wgs_of(p, 256) + 255) / 256) * (p.g.k / 64.0 + 8.0);
-}
-double mid_cost(const Problem& p) {
-  return (double)((wgs_of(p, 128) + 255) / 256) * (0.38 * p.g.k / 64.0 + 2.6);
-}
-
-// Whether the quadrant tiles take a product: 64-deep stages, two at least; an
-// addend in 16-byte rows; operand extents in 32-bit byte offsets.
-bool quad_ok(const Problem& p) {
-  const GemmArgs& g = p.g;
-  constexpr int64_t kReach = (int64_t)1 << 31;
-  auto reach = [](int64_t rows, int64_t ld) { return 2 * rows * ld < kReach; };
-  return g.k % 64 == 0 && g.k >= 128 && reach(g.m, g.lda) && reach(g.b_kn ? g.k : g.n, g.ldb) &&
-         (!g.d || (g.ldd % 8 == 0 && g.sd % 8 == 0 && g.n_lim % 8 == 0 && aligned16(g.d) &&
-                   reach(g.m_lim, g.ldd)));
+int launch_group_typed(const std::vector<const Problem*>& ps, int tile, hipStream_t stream) {
+  switch (tile) {
+    case kBig: return launch_tile_group<T, OUT_T, MODE, BigTile>(ps, stream);
+    case kMid: return launch_tile_group<T, OUT_T, MODE, MidTile>(ps, stream);
+    default: return launch_tile_group<T, OUT_T, MODE, SmallTile>(ps, stream);
+  }
 }
 
 template <typename T, typename OUT_T, int MODE>
 int launch_typed(const Problem& p, hipStream_t stream) {
-  // Depths that are an odd multiple of 32 (and what quad_ok refuses) run 32-deep
+  // Depths that are an odd multiple of 32 (and what tiles_ok refuses) run 32-deep
   // stages in a ring of four.
   using Big32 = PipeCfg<256, 256, 4, 4, 4, 32>;
   using Mid32 = PipeCfg<128, 128, 2, 2, 4, 32>;
@@ -1598,11 +1814,15 @@ int launch_typed(const Problem& p, hipStream_t stream) {
     set_error("gemm: a [k, n] B operand needs k to be a multiple of 32");
     return kInvalid;
   }
-  if (quad_ok(p))
-    return big_cost(p) <= mid_cost(p) ? launch_quad<T, OUT_T, MODE, BigTile>(p, stream)
-                                      : launch_quad<T, OUT_T, MODE, MidTile>(p, stream);
+  if (tiles_ok(p)) {
+    switch (best_tile(p)) {
+      case kBig: return launch_tile<T, OUT_T, MODE, BigTile>(p, stream);
+      case kMid: return launch_tile<T, OUT_T, MODE, MidTile>(p, stream);
+      default: return launch_tile<T, OUT_T, MODE, SmallTile>(p, stream);
+    }
+  }
   if (k32)
-    return big_cost(p) <= mid_cost(p) ? launch_pipe<T, OUT_T, MODE, Big32>(p, stream)
+    return product_time(p, kBig) <= product_time(p, kMid) ? launch_pipe<T, OUT_T, MODE, Big32>(p, stream)
                                       : launch_pipe<T, OUT_T, MODE, Mid32>(p, stream);
   if (wgs_of(p, 128) >= 512) return launch_cfg<T, OUT_T, 128, 128, 2, 2, MODE>(p, stream);
   return launch_cfg<T, OUT_T, 64, 64, 2, 2, MODE>(p, stream);
@@ -1644,38 +1864,49 @@ int launch(const Problem& p, hipStream_t stream) {
   return kInvalid;
 }
 
-// Whether one grouped launch beats one launch per product, and on which tile, in
-// the units of big_cost. Alone, each product takes its better tile; grouped, the
-// tiles of all of them fill the CUs longest first, which costs the longest tile
-// where they are one round, else their total work over the CUs plus about half a
-// round of the shortest tiles. A launch of one round or less, and each of two
-// independent products of one run (pair), also costs its ramp and drain (kRamp,
-// about 6 us).
+// Whether one grouped launch beats one launch per product, and on which tile (-1:
+// none), in the units of tile_time. Alone, each product takes its better tile;
+// grouped, the tiles of all of them fill the CUs longest first, which costs the
+// longest tile where they are one round, else their total work over the CUs plus
+// about half a round of the shortest tiles. A launch of one round or less, and each
+// of two independent products of one run (pair), also costs its ramp and drain
+// (kRamp, about 6 us).
 constexpr double kRamp = 5.3;
 
-GroupTile group_plan(const std::vector<const Problem*>& ps, bool pair) {
-  double separate = 0.0, ramp = 0.0, work[2] = {}, longest[2] = {}, shortest[2] = {1e300, 1e300};
-  int64_t wgs[2] = {};
+int64_t shortest_depth(const std::vector<const Problem*>& ps) {
+  int64_t k = INT64_MAX;
+  for (const Problem* p : ps) k = std::min<int64_t>(k, p->g.k);
+  return k;
+}
+
+int group_plan(const std::vector<const Problem*>& ps, bool pair) {
+  double separate = 0.0, ramp = 0.0;
   for (const Problem* p : ps) {
-    const double k = p->g.k / 64.0, tile[2] = {k + 8.0, 0.38 * k + 2.6};
-    const double alone[2] = {big_cost(*p), mid_cost(*p)};
-    const int best = alone[0] <= alone[1] ? 0 : 1;
-    const bool ramps = pair || wgs_of(*p, best ? 128 : 256) <= 256;
+    const int tile = best_tile(*p);
+    const bool ramps = pair || wgs_of(*p, kTileSide[tile]) <= 256;
     if (ramps) ramp = kRamp;
-    separate += (ramps ? kRamp : 0.0) + alone[best];
-    for (int c = 0; c < 2; ++c) {
-      const int64_t n = wgs_of(*p, c ? 128 : 256);
-      wgs[c] += n;
-      work[c] += tile[c] * (double)n / 256.0;
-      longest[c] = std::max(longest[c], tile[c]);
-      shortest[c] = std::min(shortest[c], tile[c]);
+    separate += (ramps ? kRamp : 0.0) + product_time(*p, tile);
+  }
+  int best = -1;
+  for (int c = kBig; c <= kSmall; ++c) {
+    double work = 0.0, longest = 0.0, shortest = 1e300;
+    int64_t wgs = 0;
+    for (const Problem* p : ps) {
+      const int64_t n = wgs_of(*p, kTileSide[c]);
+      const double one = tile_time(c, p->g.k);
+      wgs += n;
+      work += one * (double)n / 256.0;
+      longest = std::max(longest, one);
+      shortest = std::min(shortest, one);
+    }
+    if (!tile_fits(c, wgs) || (c != kSmall && shortest_depth(ps) < 128)) continue;
+    const double total = ramp + (wgs <= 256 ? longest : std::max(longest, work + 0.5 * shortest));
+    if (total < separate) {
+      separate = total;
+      best = c;
     }
   }
-  double total[2];
-  for (int c = 0; c < 2; ++c)
-    total[c] = ramp + (wgs[c] <= 256 ? longest[c] : std::max(longest[c], work[c] + 0.5 * shortest[c]));
-  if (std::min(total[0], total[1]) >= separate) return kNoGroup;
-  return total[1] < total[0] ? kGroupMid : kGroupBig;
+  return best;
 }
 
 // Independent products in as few launches as possible: one grouped launch when
@@ -1689,20 +1920,20 @@ std::vector<const Problem*> live_products(const std::vector<const Problem*>& ps)
   return live;
 }
 
-GroupTile groups(const std::vector<const Problem*>& live, bool pair = false) {
+int groups(const std::vector<const Problem*>& live, bool pair = false) {
   bool together = live.size() >= 2 && live.size() <= (size_t)kMaxGroup;
   for (const Problem* p : live)
     together = together && p->elem == live[0]->elem && p->out_mode == live[0]->out_mode &&
-               p->g.b_kn == live[0]->g.b_kn && !p->g.d == !live[0]->g.d && quad_ok(*p) &&
+               p->g.b_kn == live[0]->g.b_kn && !p->g.d == !live[0]->g.d && tiles_ok(*p) &&
                p->batch <= INT32_MAX && operands_ok(p->g) &&
                !(p->g.b_kn && (p->g.n % 8 || p->g.sym));
-  return together ? group_plan(live, pair) : kNoGroup;
+  return together ? group_plan(live, pair) : -1;
 }
 
 int launch_group(const std::vector<const Problem*>& ps, hipStream_t stream, bool pair = false) {
   const std::vector<const Problem*> live = live_products(ps);
-  const GroupTile tile = groups(live, pair);
-  if (tile == kNoGroup) {
+  const int tile = groups(live, pair);
+  if (tile < 0) {
     for (const Problem* p : live) DIONW_TRY(launch(*p, stream));
     return kOk;
   }
@@ -2073,7 +2304,7 @@ int walk_groups(const std::vector<std::vector<Problem>>& progs, bool issue, hipS
     for (size_t pos = 0; pos < prog.size(); ++pos) {
       if (prog[pos].with_next && pos + 1 < prog.size() && runs.size() == 1) {
         const std::vector<const Problem*> pair{&prog[pos], &prog[pos + 1]};
-        if (groups(live_products(pair), true) != kNoGroup) {
+        if (groups(live_products(pair), true) >= 0) {
           *launches += 1;
           if (issue) DIONW_TRY(launch_group(pair, stream, true));
           ++pos;
@@ -2083,7 +2314,7 @@ int walk_groups(const std::vector<std::vector<Problem>>& progs, bool issue, hipS
       std::vector<const Problem*> ps;
       for (int j : runs) ps.push_back(&progs[j][pos]);
       const std::vector<const Problem*> live = live_products(ps);
-      *launches += groups(live) != kNoGroup ? 1 : (int64_t)live.size();
+      *launches += groups(live) >= 0 ? 1 : (int64_t)live.size();
       if (issue) DIONW_TRY(launch_group(ps, stream));
     }
   }

@@ -14,6 +14,7 @@ import pytest
 import torch
 
 from dionw_amd._kernels import gemm_nt
+from dionw_amd.newton_schulz import NewtonSchulz, newton_schulz_fn
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -45,7 +46,10 @@ def _check(got: torch.Tensor, product: torch.Tensor, scale: torch.Tensor, k: int
     (40, 264, 520, 192, True, 8),    # a few rows and columns past,
     (40, 385, 640, 128, True, 0),    # and half of the last tile used
     (40, 392, 633, 256, False, 0),
-    (64, 513, 248, 64, False, 0),    # one stage: the 32-deep kernel
+    (64, 513, 248, 64, False, 0),    # one stage and many tiles: the 32-deep kernel
+    (2, 100, 72, 64, True, 8),       # 64x64 tiles: one stage,
+    (1, 65, 130, 576, True, 0),      # more stages than the ring holds,
+    (3, 40, 24, 1024, False, 8),     # less than a tile
 ])
 def test_product_at_tile_edges(batch, m, n, k, addend, pad, dtype) -> None:
     print(f"{batch} x {m}x{n}x{k} addend {addend} pad {pad} {dtype}", flush=True)
@@ -68,7 +72,7 @@ def test_product_at_tile_edges(batch, m, n, k, addend, pad, dtype) -> None:
 
 
 @pytest.mark.parametrize(("batch", "n", "k", "addend"), [
-    (1, 64, 128, True), (2, 136, 192, True), (1, 200, 256, False), (3, 384, 384, True),
+    (1, 64, 128, True), (1, 64, 64, True), (2, 136, 192, True), (1, 200, 256, False), (3, 384, 384, True),
     (40, 264, 128, False), (40, 512, 512, True), (40, 392, 448, True),
 ])
 def test_symmetric_product_at_tile_edges(batch, n, k, addend) -> None:
@@ -86,3 +90,23 @@ def test_symmetric_product_at_tile_edges(batch, n, k, addend) -> None:
     full = gemm_nt(a, a, d=d, alpha=2.0, beta=beta)
     assert torch.equal(torch.triu(got), torch.triu(full))
     assert torch.equal(got, got.mT)
+
+
+@pytest.mark.parametrize(("blocks", "r", "c"), [
+    (1, 64, 72), (2, 128, 200), (60, 192, 264), (3, 320, 1000), (40, 512, 776),
+])
+def test_left_products_read_the_iterate_as_it_lies(blocks: int, r: int, c: int) -> None:
+    """The products that read X as a [k, n] operand, on each tile and with columns
+    that end inside a tile: five Keller steps against the same polynomials in
+    float64 (bf16 rounding: within 0.03, as the quintics' oracle is)."""
+    print(f"{blocks} x {r}x{c}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(r + c)
+    x = torch.randn(blocks, r, c, device=DEV, generator=g)
+    got = newton_schulz_fn(NewtonSchulz.KELLER_TRITON)(x, 1e-8).double()
+    y = x.double()
+    y = y / y.flatten(1).norm(dim=1).view(-1, 1, 1)
+    for _ in range(5):
+        gram = torch.matmul(y, y.mT.contiguous())
+        y = 3.4445 * y + torch.matmul(2.0315 * torch.matmul(gram, gram) - 4.7750 * gram, y)
+    for b in range(blocks):
+        assert (got[b] - y[b]).norm() <= 0.03 * y[b].norm(), f"block {b}"
