@@ -50,12 +50,12 @@ from dionw_amd.newton_schulz import (
     NewtonSchulzCall,
     group_launches,
     newton_schulz_call,
-    padded_sides,
     prepared_inputs,
     prepared_orientations,
     run_newton_schulz,
     run_newton_schulz_call,
     run_newton_schulz_group,
+    tile_sides,
 )
 
 __all__ = ["ACTIVE_RUNS", "MAX_RUN_ELEMENTS", "PROFILE_REGION", "RunQueue", "step_run"]
@@ -292,10 +292,10 @@ def _queued_name(name: str) -> bool:
 
 def _ns_bytes(ortho: HipOrthogonalize, blocks: int, k: int, cols: int) -> int:
     """Bytes of a fused run's Newton-Schulz buffers (inputs, output, workspace)."""
-    p_pad, j_pad = padded_sides(k, cols)
+    p_pad, j_pad = sides = tile_sides(blocks, k, cols)
     r, c = min(p_pad, j_pad), max(p_pad, j_pad)
     work = int(_lib.library().dionw_newton_schulz_workspace(ortho.lib_kind, blocks, r, c))
-    inputs = sum(prepared_orientations(k, cols))
+    inputs = sum(prepared_orientations(k, cols, sides))
     return inputs * 2 * blocks * p_pad * j_pad + 2 * blocks * k * cols + work
 
 
@@ -356,10 +356,11 @@ def step_run(
         idx_ptr = None if idx is None else idx.data_ptr()
         if fused:
             # Only the orientations the iteration reads are written.
+            sides = tile_sides(blocks, k, cols)
             xr, xt = prepared_inputs(ortho, device, blocks, k, cols, "ns_xr" + own,
-                                     "ns_xt" + own)
+                                     "ns_xt" + own, sides)
             _lib.call("dionw_prepare_ns_input", grads, count, momentum.data_ptr(), idx_ptr,
-                      den.data_ptr(), blocks, rows, cols, k, *padded_sides(k, cols), mu,
+                      den.data_ptr(), blocks, rows, cols, k, *sides, mu,
                       int(nesterov), 1, ortho.elem, None if xr is None else xr.data_ptr(),
                       None if xt is None else xt.data_ptr(), stream)
         else:
@@ -372,12 +373,12 @@ def step_run(
         orthogonal = _workspace.buffer(device, "ns_out" + own, (blocks, k, cols), torch.bfloat16)
         if queue is not None:
             call = newton_schulz_call(ortho, blocks, k, cols, xr, xt, orthogonal,
-                                      "ns_workspace" + own)
+                                      "ns_workspace" + own, sides)
             queue.add(call, partial(_finish_run, run, bucket, positions, group, orthogonal, idx,
                                     slot, step), nbytes, stream, device)
             return
         with region(ORTHOGONALIZE_REGION):
-            run_newton_schulz(ortho, blocks, k, cols, xr, xt, orthogonal, stream)
+            run_newton_schulz(ortho, blocks, k, cols, xr, xt, orthogonal, stream, sides)
     else:
         with region(ORTHOGONALIZE_REGION):
             orthogonal = ortho(raw, NEWTON_SCHULZ_EPS)
