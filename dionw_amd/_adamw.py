@@ -57,8 +57,11 @@ def adamw_step(group: dict[str, Any], state: ParamState) -> None:
             raise TypeError(f"the HIP AdamW takes float32 parameters, got {param.dtype}")
         data = param.data
         m, v = entry[EXP_AVG_STATE], entry[EXP_AVG_SQ_STATE]
-        grad = grad.to(torch.float32)
-        if not all(same_dense_layout(t, data) for t in (grad, m, v)):
+        if grad.dtype is not torch.float32:
+            grad = grad.to(torch.float32)
+        row_major = (data.is_contiguous() and grad.is_contiguous() and m.is_contiguous()
+                     and v.is_contiguous() and data.shape == grad.shape == m.shape == v.shape)
+        if not row_major and not all(same_dense_layout(t, data) for t in (grad, m, v)):
             # Mixed layouts: step row-major copies and write them back.
             flat = [t.contiguous() for t in (data, m, v)]
             copies.extend(zip((data, m, v), flat, strict=True))

@@ -189,7 +189,9 @@ def int64_array(values: Sequence[int]) -> ctypes.Array[ctypes.c_int64]:
 
 def stream_handle(device: torch.device | None = None) -> int:
     """The raw HIP stream of torch's current stream on ``device``."""
-    return torch.cuda.current_stream(device).cuda_stream
+    index = None if device is None else device.index
+    return int(torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index))
 
 
 def elem_code(dtype: torch.dtype) -> int:

@@ -112,7 +112,8 @@ def _make_run(bucket: Bucket, positions: list[int] | range) -> _Run:
         if grad is None:
             raise RuntimeError("every parameter of a Dion run needs a gradient")
         # Channels-last (or otherwise strided) tensors go through row-major copies.
-        grads.append(grad.to(torch.float32).contiguous())
+        plain = grad.dtype is torch.float32 and grad.is_contiguous()
+        grads.append(grad if plain else grad.to(torch.float32).contiguous())
         if param.is_contiguous():
             params.append(param.data)
         else:
@@ -221,10 +222,10 @@ class RunQueue:
                             or self._bytes + nbytes > QUEUE_BYTES):
             self.flush()
         own = f"#{len(self._calls)}"
-        kept = _workspace.named_bytes(device, stream, _queued_name)
+        suffix = own[1:]
         mine = _workspace.named_bytes(device, stream,
-                                      lambda name: name.partition("#")[2] == own[1:])
-        others = kept - mine
+                                      lambda name: name.partition("#")[2] == suffix)
+        others = _workspace.named_bytes(device, stream, _queued_name) - mine
         if others > 0 and others + max(mine, nbytes) > QUEUE_BYTES:
             self.flush()
             _workspace.release_named(device, stream, _queued_name)
@@ -254,7 +255,8 @@ class RunQueue:
             return
         calls, finish, stream, device = self._calls, self._finish, self._stream, self._device
         self._calls, self._finish, self._bytes, self._stream = [], [], 0, None
-        grouped = len(calls) > 1 and group_launches(calls) < sum(group_launches([c]) for c in calls)
+        alone = [group_launches([c]) for c in calls] if len(calls) > 1 else []
+        grouped = len(calls) > 1 and group_launches(calls) < sum(alone)
         lanes = _lanes(calls, grouped)
         if len(lanes) == 1:
             _run_lane(calls, finish, lanes[0], grouped, stream)
@@ -263,19 +265,21 @@ class RunQueue:
         side = _side_stream(device)
         side.wait_stream(main)
         for lane, lane_stream in zip(lanes, (main, side)):
+            shared = grouped and len(lane) > 1 and (
+                group_launches([calls[i] for i in lane]) < sum(alone[i] for i in lane))
             with torch.cuda.stream(lane_stream):
-                _run_lane(calls, finish, lane, grouped, lane_stream.cuda_stream)
+                _run_lane(calls, finish, lane, shared, lane_stream.cuda_stream)
         main.wait_stream(side)
 
 
 def _run_lane(calls: list[NewtonSchulzCall], finish: list[Callable[[], None]], lane: list[int],
               grouped: bool, stream: int) -> None:
-    """The calls ``lane`` of the queue, then (or each followed by) their runs' passes."""
+    """The calls ``lane`` of the queue, grouped and then their runs' passes, or each
+    followed by its run's."""
     region = PROFILE_REGION.get()
-    mine = [calls[i] for i in lane]
-    if grouped and len(mine) > 1 and group_launches(mine) < sum(group_launches([c]) for c in mine):
+    if grouped:
         with region(ORTHOGONALIZE_REGION):
-            run_newton_schulz_group(mine, stream)
+            run_newton_schulz_group([calls[i] for i in lane], stream)
         for i in lane:
             finish[i]()
         return

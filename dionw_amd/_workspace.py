@@ -23,15 +23,23 @@ from collections.abc import Callable
 
 import torch
 
+from dionw_amd import _lib
+
 __all__ = ["buffer", "release", "release_named", "held_bytes", "named_bytes", "share", "tensors"]
 
 _ALIGN = 256
 _BUFFERS: dict[tuple[torch.device, int, str], torch.Tensor] = {}
+# The last view taken of each buffer: (shape, dtype, buffer, view). A step asks for the
+# same views every time, and making one costs four tensor operations.
+_VIEWS: dict[tuple[torch.device, int, str],
+             tuple[tuple[int, ...], torch.dtype, torch.Tensor, torch.Tensor]] = {}
 
 
 def _resolved(device: torch.device | str) -> torch.device:
     """``device`` with its index filled in: ``cuda`` means the current GPU, so
     that ``cuda`` and ``cuda:0`` name the same buffers when GPU 0 is current."""
+    if type(device) is torch.device and device.index is not None:
+        return device
     device = torch.device(device)
     if device.type == "cuda" and device.index is None:
         return torch.device("cuda", torch.cuda.current_device())
@@ -41,7 +49,7 @@ def _resolved(device: torch.device | str) -> torch.device:
 def _stream_of(device: torch.device) -> int:
     if device.type != "cuda":
         return 0
-    return torch.cuda.current_stream(device).cuda_stream
+    return _lib.stream_handle(device)
 
 
 def _retire(store: torch.Tensor, stream: int) -> None:
@@ -57,24 +65,35 @@ def buffer(device: torch.device, name: str, shape: tuple[int, ...], dtype: torch
     (torch's current stream on ``device`` when None); uninitialized."""
     device = _resolved(device)
     stream = _stream_of(device) if stream is None else stream
-    numel = math.prod(shape)
-    nbytes = max(numel * torch.empty((), dtype=dtype).element_size(), 1)
     key = (device, stream, name)
     store = _BUFFERS.get(key)
+    held = _VIEWS.get(key)
+    if held is not None and held[0] == shape and held[1] is dtype and held[2] is store:
+        return held[3]
+    numel = math.prod(shape)
+    nbytes = max(numel * dtype.itemsize, 1)
     if store is None or store.numel() < nbytes:
         if store is not None:
+            _VIEWS.pop(key, None)
             _retire(store, stream)
         store = torch.empty(((nbytes + _ALIGN - 1) // _ALIGN) * _ALIGN, dtype=torch.uint8,
                             device=device)
         _BUFFERS[key] = store
-    return store[:nbytes].view(dtype)[:numel].view(shape)
+    view = store[:nbytes].view(dtype)[:numel].view(shape)
+    _VIEWS[key] = (tuple(shape), dtype, store, view)
+    return view
+
+
+def _drop(key: tuple[torch.device, int, str]) -> None:
+    _VIEWS.pop(key, None)
+    _retire(_BUFFERS.pop(key), key[1])
 
 
 def release(device: torch.device | None = None) -> None:
     """Drop the scratch buffers (of ``device``, or all)."""
     device = None if device is None else _resolved(device)
     for key in [k for k in _BUFFERS if device is None or k[0] == device]:
-        _retire(_BUFFERS.pop(key), key[1])
+        _drop(key)
 
 
 def named_bytes(device: torch.device, stream: int, match: Callable[[str], bool]) -> int:
@@ -88,7 +107,7 @@ def release_named(device: torch.device, stream: int, match: Callable[[str], bool
     """Drop the buffers of ``device`` and ``stream`` whose names ``match``."""
     device = _resolved(device)
     for key in [k for k in _BUFFERS if k[0] == device and k[1] == stream and match(k[2])]:
-        _retire(_BUFFERS.pop(key), key[1])
+        _drop(key)
 
 
 def held_bytes(device: torch.device | None = None) -> int:

@@ -269,7 +269,6 @@ class OptimizerIntegratedEMA:
             raise TypeError(f"a saved {type(self.optimizer).__name__} EMA shadow is not a tensor")
         self._place(param, self.optimizer.state[param], saved, bool(initialized))
 
-    @torch.no_grad()
     def update_param(self, param: Tensor) -> None:
         """Queue or stage one parameter's due update (parameters without
         optimizer state are skipped)."""
@@ -280,12 +279,13 @@ class OptimizerIntegratedEMA:
             if id(param) in self._fused:
                 entry[EMA_PENDING] = False
                 return
-            if EMA_SHADOW not in entry:
-                self._place(param, entry, None, False)
-            if not self._on_gpu:
-                if id(param) not in self._staged:
-                    self._stage([(param, entry)])
-                return
+            with torch.no_grad():
+                if EMA_SHADOW not in entry:
+                    self._place(param, entry, None, False)
+                if not self._on_gpu:
+                    if id(param) not in self._staged:
+                        self._stage([(param, entry)])
+                    return
             restart = self._now.from_live or not entry[EMA_INITIALIZED]
             queue = self._copies if restart else self._lerps
             queue[0].append(entry[EMA_SHADOW])
