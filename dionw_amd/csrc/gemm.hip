@@ -1,9 +1,9 @@
 // MFMA products of the Newton-Schulz iterations and their drivers.
 //
 // Every product is one "NT" form, C[i,j] = sum_k A[i,k] B[j,k] with both
-// operands row-major along k, computed with v_mfma_f32_32x32x16_{f16,bf16}
-// (fp32 accumulation, every element over k in order, whatever the tile) from
-// LDS-staged k tiles (64 deep; 32 deep where k is an odd multiple of 32). The epilogue forms
+// operands row-major along k, computed with v_mfma_f32_16x16x32_{f16,bf16} from
+// 64-deep LDS-staged k tiles, or v_mfma_f32_32x32x16_* where k is no multiple of 64
+// (fp32 accumulation, every element over k in order, whatever the tile). The epilogue forms
 // alpha * acc + beta * D[i,j] and rounds once to the storage type; in mode
 // kOutRoundAcc it rounds the product to the storage type first, then forms
 // alpha * bf16(acc) + beta * D and rounds again (a product stored by one
@@ -79,12 +79,18 @@ struct Mfma<_Float16> {
   __device__ static f32x16 run(vec a, vec b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }
+  __device__ static f32x4 run16(vec a, vec b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
 };
 template <>
 struct Mfma<__bf16> {
   typedef bf16x8 vec;
   __device__ static f32x16 run(vec a, vec b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+  __device__ static f32x4 run16(vec a, vec b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
 };
 
@@ -714,12 +720,12 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
 // ---- tiles in quadrants ------------------------------------------------------------
 //
 // The products' main kernel, for depths that are a multiple of 64. WM x WN waves;
-// the tile is 2 WM FI 32 rows by 2 WN FJ 32 columns, split into two halves each
-// way. A wave owns FI x FJ fragments of 32x32 in each of the four quadrants (rows
+// the tile is 2 WM FI 16 rows by 2 WN FJ 16 columns, split into two halves each
+// way. A wave owns FI x FJ fragments of 16x16 in each of the four quadrants (rows
 // half qi, columns half qj) and multiplies them one after the other, 0 0, 0 1,
 // 1 1, 1 0: each step changes one operand's half, whose fragments are read from
 // LDS under the MFMAs of the step before, into registers that those MFMAs free
-// k-step by k-step. So the MFMAs wait for no LDS read.
+// fragment by fragment. So the MFMAs wait for no LDS read.
 //
 // An operand's half stage (64 deep) is a slot of its own in a ring of two stages.
 // Its fragments leave LDS early (whole-depth fragments sit in registers), so the
@@ -736,19 +742,24 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
 // of a row: the epilogue moves 8 bytes per LDS access, and the mirrored store
 // reads its columns with transpose reads.
 //
-// What bounds it: the MFMA pipe and the board's power limit. At 8192^3 the pipe is
-// busy 80% of cycles (62% with one barrier per stage and every stage's loads
-// waited for one stage later, 16 waves of 64x64), at 1.36-1.5 GHz. Measured, before
-// and after, us: 8192^3 1015 / 890; 8 x 3584^3 symmetric with addend 457 / 398
-// (806 / 924 TFLOP/s); 4 x 3584 x 4096 x 3584 438 / 382; 16 x 1024^3 symmetric with
-// addend 38 / 32; 64 x 1408 x 1408 x 2048 389 / 324 (whose ragged tiles multiply
-// half). Not kept: four waves of 128x128 (442 on 8 x 3584^3 where this took 421),
-// a barrier per quadrant (421 against 398), the loads after later k-steps (+1%).
+// What bounds it: the board's power, then the MFMA pipe. On random operands in
+// registers, with nothing else running, v_mfma_f32_16x16x32_f16 sustains 1935
+// TFLOP/s and v_mfma_f32_32x32x16_f16 1640 (it reads and writes twice the
+// accumulators per product); both sum an element's k in the same order, bit for
+// bit. With the 16x16 instructions 8192^3 takes 763 us instead of 840 (1441
+// TFLOP/s, the pipe busy 80% of cycles at 1.48 GHz), 8 x 3584^3 symmetric with
+// addend 351 instead of 385, 4 x 3584 x 4096 x 3584 330 instead of 366. Against one
+// barrier per stage, 16 waves of 64x64, 32x32 instructions and every stage's loads
+// waited for one stage later: 8192^3 968 / 763, 8 x 3584^3 439 / 351, 16 x 1024^3
+// symmetric with addend 38 / 30, 64 x 1408 x 1408 x 2048 377 / 296 (whose ragged
+// tiles multiply half). Not kept: four waves of 128x128 (442 on 8 x 3584^3 where
+// eight took 421), a barrier per quadrant (421 against 398), the loads after later
+// k-steps (+1%), first tiles started at staggered times (+1 to +4%).
 template <int WM_, int WN_, int FI_, int FJ_>
 struct QuadCfg {
   static constexpr int WM = WM_, WN = WN_, FI = FI_, FJ = FJ_;
   static constexpr int waves = WM * WN, threads = waves * 64;
-  static constexpr int HM = WM * FI * 32, HN = WN * FJ * 32;  // half tile rows / columns
+  static constexpr int HM = WM * FI * 16, HN = WN * FJ * 16;  // half tile rows / columns
   static constexpr int halves = 2, BM = halves * HM, BN = halves * HN;
   static constexpr int depth = 64;
   static constexpr int a_half = HM * depth, b_half = HN * depth;   // elements of a half stage
@@ -758,8 +769,8 @@ struct QuadCfg {
   static_assert((size_t)BM * BN * 2 <= lds_bytes, "the output tile is assembled in the ring");
 };
 
-using BigTile = QuadCfg<2, 4, 2, 1>;  // 256x256, 8 waves, one workgroup per CU
-using MidTile = QuadCfg<2, 2, 1, 1>;  // 128x128, 4 waves, two workgroups per CU
+using BigTile = QuadCfg<2, 4, 4, 2>;  // 256x256, 8 waves, one workgroup per CU
+using MidTile = QuadCfg<2, 2, 2, 2>;  // 128x128, 4 waves, two workgroups per CU
 
 // The output tile in LDS: rows of BN elements, 16-byte chunk ch of row r at
 // ch ^ epi_swz(r).
@@ -772,7 +783,7 @@ template <int BN>
 __device__ __forceinline__ int epi_off(int r, int ch) { return r * BN + ((ch ^ epi_swz<BN>(r)) << 3); }
 
 template <typename T, typename OUT_T, int MODE, typename CFG, bool ADD>
-__device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x16 (&acc)[CFG::halves * CFG::FI][CFG::halves * CFG::FJ],
+__device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CFG::halves * CFG::FI][CFG::halves * CFG::FJ],
                                               int64_t bidx, int m0, int n0, int wave, int lane,
                                               bool skip1x, bool skipx1, bool diag_tile,
                                               unsigned char* smem) {
@@ -782,40 +793,37 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x16 (&acc)[C
   typedef T t4 __attribute__((ext_vector_type(4)));
   const int wm = wave / CFG::WN, wn = wave % CFG::WN;
   const int tid = wave * 64 + lane;
-  const int lrow = lane & 31, lk = lane >> 5;
   OUT_T* tile = reinterpret_cast<OUT_T*>(smem);
   OUT_T* C = g.c ? reinterpret_cast<OUT_T*>(g.c) + bidx * g.sc : nullptr;
   OUT_T* CT = g.ct ? reinterpret_cast<OUT_T*>(g.ct) + bidx * g.sct : nullptr;
   OUT_T* CD = g.c_diag ? reinterpret_cast<OUT_T*>(g.c_diag) + bidx * g.sc : nullptr;
   __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt(0) lgkmcnt(0): the addend has landed
   __builtin_amdgcn_s_barrier();
+  // Each lane holds 4 consecutive columns of one row of every 16x16 fragment.
+  const int G = lane >> 4, i16 = lane & 15;
 #pragma unroll
   for (int i = 0; i < CFG::halves * CFG::FI; ++i) {
     if (i >= CFG::FI && skip1x) continue;
+    const int r = (i / CFG::FI) * CFG::HM + (wm * CFG::FI + i % CFG::FI) * 16 + i16;
+    OUT_T* at[CFG::halves * CFG::FJ];
+    t4 d[CFG::halves * CFG::FJ];
+#pragma unroll
+    for (int j = 0; j < CFG::halves * CFG::FJ; ++j) {
+      const int ch = ((j / CFG::FJ) * CFG::HN + (wn * CFG::FJ + j % CFG::FJ) * 16) / 8 + (G >> 1);
+      at[j] = tile + epi_off<BN>(r, ch) + 4 * (G & 1);
+      if (ADD) d[j] = *reinterpret_cast<const t4*>(at[j]);
+    }
 #pragma unroll
     for (int j = 0; j < CFG::halves * CFG::FJ; ++j) {
       if (j >= CFG::FJ && skipx1) continue;
       if (i >= CFG::FI && j < CFG::FJ && diag_tile) continue;
-      const int r = (i / CFG::FI) * CFG::HM + (wm * CFG::FI + i % CFG::FI) * 32 + lrow;
-      const int ch0 = ((j / CFG::FJ) * CFG::HN + (wn * CFG::FJ + j % CFG::FJ) * 32) / 8;
-      t4 d[4];
-      if (ADD) {
+      o4 v;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          d[q] = *reinterpret_cast<const t4*>(reinterpret_cast<const T*>(tile) +
-                                              epi_off<BN>(r, ch0 + q) + 4 * lk);
+      for (int k = 0; k < 4; ++k) {
+        const float p = product_value<OUT_T, MODE>(acc[i][j][k]);
+        v[k] = round_out<OUT_T, MODE>(ADD ? axpby(g.alpha, p, g.beta, (float)d[j][k]) : g.alpha * p);
       }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        o4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float p = product_value<OUT_T, MODE>(acc[i][j][4 * q + e]);
-          v[e] = round_out<OUT_T, MODE>(ADD ? axpby(g.alpha, p, g.beta, (float)d[q][e])
-                                                        : g.alpha * p);
-        }
-        *reinterpret_cast<o4*>(tile + epi_off<BN>(r, ch0 + q) + 4 * lk) = v;
-      }
+      *reinterpret_cast<o4*>(at[j]) = v;
     }
   }
   __syncthreads();
@@ -830,7 +838,6 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x16 (&acc)[C
   const bool vec_rows = (g.ldc % 8 == 0) && (g.sc % 8 == 0) &&
                         ((reinterpret_cast<uintptr_t>(g.c) | reinterpret_cast<uintptr_t>(g.c_diag)) & 15) == 0;
   const bool vec_cols = g.ldct % 8 == 0 && g.sct % 8 == 0 && (reinterpret_cast<uintptr_t>(g.ct) & 15) == 0;
-  const int G = lane >> 4, i16 = lane & 15;
   if (m0 + BM <= g.m_lim && n0 + BN <= g.n_lim && vec_rows && vec_cols) {
     // A whole tile: every LDS read of a batch is issued before its first store. A
     // diagonal tile stores its 8x8 blocks on and above the diagonal as they lie and
@@ -945,6 +952,14 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x16 (&acc)[C
   }
 }
 
+// B as [k, n]: 16-byte chunk ch of k-row r of N columns sits at ch ^ kn_swz(r), so that
+// the 4 k-rows of one 16-lane group's transpose read and the 4 of its neighbour, 8 rows
+// on, fall on 16 distinct 16-byte bank groups.
+template <int N>
+__device__ __forceinline__ int kn_swz(int r) {
+  return (N >= 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1)) | (2 * ((r >> 3) & 1));
+}
+
 template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
 __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
 #ifdef __HIP_DEVICE_COMPILE__  // the host pass has no buffer-resource type
@@ -988,8 +1003,7 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
       a_off[h][j] = (uint32_t)min(h * HM + row, g.m - 1 - m0) * (uint32_t)(2 * g.lda) + 16 * ch;
       if (BKN) {
         constexpr int NCH = HN / 8;
-        const int krow = pos / NCH;
-        const int c = (pos % NCH) ^ (NCH >= 16 ? 4 * (krow & 3) : 4 * ((krow >> 1) & 1));
+        const int krow = pos / NCH, c = (pos % NCH) ^ kn_swz<HN>(krow);
         b_off[h][j] = (uint32_t)krow * (uint32_t)(2 * g.ldb) +
                       2 * (uint32_t)min(h * HN + c * 8, g.n - 8 - n0);
       } else {
@@ -1025,7 +1039,7 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
   constexpr int D_SLOTS = BM / SLOT_ROWS;  // 8: every slot; 4: the A slots
   static_assert(CFG::a_half == CFG::b_half && (D_SLOTS == 8 || D_SLOTS == 4), "slot layout");
   const T* D = ADD ? reinterpret_cast<const T*>(g.d) + bidx * g.sd + (int64_t)m0 * g.ldd + n0 : nullptr;
-  const uint32_t d_bytes = ADD ? (uint32_t)(2 * ((g.m_lim - 1 - m0) * g.ldd + g.n_lim - n0)) : 0;
+  const uint32_t d_bytes = ADD ? (uint32_t)(2 * ((g.m - 1 - m0) * g.ldd + g.n - n0)) : 0;
   const auto d_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)D, 0, d_bytes, 0x00020000);
   auto load_d = [&](int slot) {
 #pragma unroll
@@ -1033,80 +1047,73 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
       const int pos = (j * W + wave) * 64 + lane;
       const int row = slot * SLOT_ROWS + pos / (BN / 8);
       const int c = ((pos % (BN / 8)) ^ epi_swz<BN>(row)) * 8;
-      const uint32_t off = (uint32_t)min(row, g.m_lim - 1 - m0) * (uint32_t)(2 * g.ldd) +
-                           2 * (uint32_t)min(c, g.n_lim - 8 - n0);
+      const uint32_t off = (uint32_t)min(row, g.m - 1 - m0) * (uint32_t)(2 * g.ldd) +
+                           2 * (uint32_t)min(c, g.n - 8 - n0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           d_rsrc, (lds_ptr_t)(lds_a + slot * CFG::a_half + (j * W + wave) * 512), 16, off, 0, 0, 0);
     }
   };
 
-  const int lrow = lane & 31, lk = lane >> 5;
-  const int sw = (lrow >> 1) & 7;
-  const T* a_rd[4];
-  const T* b_rd[4];
+  // A fragment is 16 rows (columns) by 32 k: lane i holds row i % 16, k 8 (i / 16) .. + 7.
+  const int G = lane >> 4, i16 = lane & 15, sw = (i16 >> 1) & 7;
+  const T* a_rd[2];
+  const T* b_rd[2];
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    a_rd[ks] = lds_a + (wm * FI * 32 + lrow) * DEPTH + (((2 * ks + lk) ^ sw) << 3);
-    b_rd[ks] = lds_b + (wn * FJ * 32 + lrow) * DEPTH + (((2 * ks + lk) ^ sw) << 3);
+  for (int ks = 0; ks < 2; ++ks) {
+    a_rd[ks] = lds_a + (wm * FI * 16 + i16) * DEPTH + (((4 * ks + G) ^ sw) << 3);
+    b_rd[ks] = lds_b + (wn * FJ * 16 + i16) * DEPTH + (((4 * ks + G) ^ sw) << 3);
   }
-  // BKN: chunk ch of k-row r of a half sits at ch ^ (4 (r % 4)) (128 columns) or
-  // ch ^ (4 (r / 2 % 2)) (64 columns).
-  const int G = lane >> 4, i16 = lane & 15;
-  const T* b_kn[FJ];
+  const T* b_kn[FJ];  // BKN: a lane's place in the transpose reads
 #pragma unroll
   for (int j = 0; j < FJ; ++j) {
-    const int col = (wn * FJ + j) * 32 + 16 * (G & 1) + 4 * (i16 & 3);
-    const int kr = i16 >> 2;  // k-row of the lane, modulo 4
-    const int x = HN >= 128 ? 4 * kr : 4 * (kr >> 1);
-    b_kn[j] = lds_b + (8 * (G >> 1) + kr) * HN + (((col >> 3) ^ x) << 3) + (col & 7);
+    const int col = (wn * FJ + j) * 16 + 4 * (i16 & 3), kr = 8 * G + (i16 >> 2);
+    b_kn[j] = lds_b + kr * HN + (((col >> 3) ^ kn_swz<HN>(kr)) << 3) + (col & 7);
   }
-  auto read_a = [&](V (&f)[FI][4], int ks, int buf, int h) {
-#pragma unroll
-    for (int i = 0; i < FI; ++i)
-      f[i][ks] = *reinterpret_cast<const V*>(a_rd[ks] + (2 * buf + h) * CFG::a_half + i * 32 * DEPTH);
+  auto read_a = [&](V (&f)[FI][2], int ks, int i, int buf, int h) {
+    f[i][ks] = *reinterpret_cast<const V*>(a_rd[ks] + (2 * buf + h) * CFG::a_half + i * 16 * DEPTH);
   };
-  auto read_b = [&](V (&f)[FJ][4], int ks, int buf, int h) {
-#pragma unroll
-    for (int j = 0; j < FJ; ++j) {
-      if (BKN) {
-        const T* p = b_kn[j] + (2 * buf + h) * CFG::b_half + ks * 16 * HN;
-        v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p));
-        v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p + 4 * HN));
-        f[j][ks] = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-      } else {
-        f[j][ks] = *reinterpret_cast<const V*>(b_rd[ks] + (2 * buf + h) * CFG::b_half + j * 32 * DEPTH);
-      }
+  auto read_b = [&](V (&f)[FJ][2], int ks, int j, int buf, int h) {
+    if (BKN) {
+      const T* p = b_kn[j] + (2 * buf + h) * CFG::b_half + ks * 32 * HN;
+      v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p));
+      v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p + 4 * HN));
+      f[j][ks] = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    } else {
+      f[j][ks] = *reinterpret_cast<const V*>(b_rd[ks] + (2 * buf + h) * CFG::b_half + j * 16 * DEPTH);
     }
   };
 
-  f32x16 acc[2 * FI][2 * FJ];
+  const bool diag_tile = g.sym && tm == tn;
+  const bool skip1x = m0 + HM >= g.m_lim, skipx1 = n0 + HN >= g.n_lim;
+  // Tiles that multiply every quadrant run a copy of the loop without the tests (two
+  // MFMAs, 32 cycles, lie between them).
+  auto run = [&](auto whole_) {
+  constexpr bool whole = decltype(whole_)::value;
+  const bool do01 = whole || !skipx1, do11 = whole || (!skip1x && !skipx1);
+  const bool do10 = whole || (!skip1x && !diag_tile);
+  f32x4 acc[2 * FI][2 * FJ];
 #pragma unroll
   for (int i = 0; i < 2 * FI; ++i)
 #pragma unroll
     for (int j = 0; j < 2 * FJ; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
 
-  const bool diag_tile = g.sym && tm == tn;
-  const bool skip1x = m0 + HM >= g.m_lim, skipx1 = n0 + HN >= g.n_lim;
-  const bool do01 = !skipx1, do11 = !skip1x && !skipx1, do10 = !skip1x && !diag_tile;
-
-  V a[FI][4], bx[FJ][4], by[FJ][4];
+  V a[FI][2], bx[FJ][2], by[FJ][2];
 #define QUAD_FENCE __builtin_amdgcn_sched_barrier(0);
 #define QUAD_SYNC(VM)                                                           \
   QUAD_FENCE                                                                    \
-  wait_vm<VM, 4 * FI>();                                                        \
+  wait_vm<VM, 2 * FI>();                                                        \
   __builtin_amdgcn_s_barrier();                                                 \
   QUAD_FENCE
-  // One k-step of a quadrant; the MFMA takes B first, so that a lane holds 4
-  // consecutive columns of one row.
-  auto multiply = [&](auto qi_, auto qj_, int ks, V (&b)[FJ][4]) {
+  // One row fragment of a quadrant over 32 k; the MFMA takes B first, so that a
+  // lane holds 4 consecutive columns of one row.
+  auto multiply = [&](auto qi_, auto qj_, int ks, int i, V (&b)[FJ][2]) {
     constexpr int qi = decltype(qi_)::value, qj = decltype(qj_)::value;
 #pragma unroll
-    for (int i = 0; i < FI; ++i)
-#pragma unroll
-      for (int j = 0; j < FJ; ++j)
-        acc[qi * FI + i][qj * FJ + j] = Mfma<T>::run(b[j][ks], a[i][ks], acc[qi * FI + i][qj * FJ + j]);
+    for (int j = 0; j < FJ; ++j)
+      acc[qi * FI + i][qj * FJ + j] =
+          Mfma<T>::run16(b[j][ks], a[i][ks], acc[qi * FI + i][qj * FJ + j]);
     QUAD_FENCE
   };
   using I0 = std::integral_constant<int, 0>;
@@ -1114,43 +1121,57 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
   using I2 = std::integral_constant<int, 2>;
   // One stage. b0 holds B0(kt) at entry; b1 holds B0(kt + 1) at exit.
   // tail 0: two more stages follow at least; 1: one; 2: none.
-  auto stage = [&](auto buf_, auto tail_, int kt, V (&b0)[FJ][4], V (&b1)[FJ][4]) {
+  auto stage = [&](auto buf_, auto tail_, int kt, V (&b0)[FJ][2], V (&b1)[FJ][2]) {
     constexpr int buf = decltype(buf_)::value, tail = decltype(tail_)::value;
     constexpr int dA = ADD ? L : 0, dB = D_SLOTS == 8 ? dA : 0;
+    static_assert(FI >= FJ, "a row fragment's step for every column fragment's read");
     // rows half 0 x columns half 0; B1(kt) is read
     QUAD_SYNC((tail != 2 ? 3 * L : dA + 2 * dB))
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      multiply(I0{}, I0{}, ks, b0);
-      read_b(b1, ks, buf, 1);
-      if (ks == 0) {
-        if (tail != 2) load_a(kt + 1, buf ^ 1, 1);
-        else if (dA) load_d(2 * (buf ^ 1) + 1);
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < FI; ++i) {
+        multiply(I0{}, I0{}, ks, i, b0);
+        if (i < FJ) read_b(b1, ks, i, buf, 1);
+        if (ks == 0 && i == 0) {
+          if (tail != 2) load_a(kt + 1, buf ^ 1, 1);
+          else if (dA) load_d(2 * (buf ^ 1) + 1);
+        }
+        QUAD_FENCE
       }
-      QUAD_FENCE
     }
     // 0 x 1; A1(kt) replaces A0(kt)
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (do01) multiply(I0{}, I1{}, ks, b1);
-      read_a(a, ks, buf, 1);
-      if (ks == 0) {
-        if (tail == 0) load_b(kt + 2, buf, 0);
-        else if (dB) load_d(4 + 2 * buf);
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < FI; ++i) {
+        if (do01) multiply(I0{}, I1{}, ks, i, b1);
+        read_a(a, ks, i, buf, 1);
+        if (ks == 0 && i == 0) {
+          if (tail == 0) load_b(kt + 2, buf, 0);
+          else if (dB) load_d(4 + 2 * buf);
+        }
+        QUAD_FENCE
       }
-      QUAD_FENCE
     }
     // 1 x 1; B0(kt + 1) replaces B1(kt)
     if (tail != 2 || ADD) {
       QUAD_SYNC((tail == 0 ? 3 * L : tail == 1 ? 2 * L + dB : 63))
     }
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (do11) multiply(I1{}, I1{}, ks, b1);
-      if (tail != 2) read_b(b1, ks, buf ^ 1, 0);
-      if (ks == 0) {
-        if (tail == 0) load_a(kt + 2, buf, 0);
-        else if (dA) load_d(2 * buf);
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < FI; ++i) {
+        if (do11) multiply(I1{}, I1{}, ks, i, b1);
+        if (ks == 0 && i == 0) {
+          if (tail == 0) load_a(kt + 2, buf, 0);
+          else if (dA) load_d(2 * buf);
+        }
+        QUAD_FENCE
+      }
+      if (tail != 2) {
+#pragma unroll
+        for (int j = 0; j < FJ; ++j) read_b(b1, ks, j, buf ^ 1, 0);
       }
       QUAD_FENCE
     }
@@ -1160,22 +1181,29 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
       load_d(2 * buf + 1);
     }
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (do10) multiply(I1{}, I0{}, ks, b0);
-      if (tail != 2) read_a(a, ks, buf ^ 1, 0);
-      if (ks == 0) {
-        if (tail == 0) load_b(kt + 2, buf, 1);
-        else if (dB) load_d(5 + 2 * buf);
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int i = 0; i < FI; ++i) {
+        if (do10) multiply(I1{}, I0{}, ks, i, b0);
+        if (tail != 2) read_a(a, ks, i, buf ^ 1, 0);
+        if (ks == 0 && i == 0) {
+          if (tail == 0) load_b(kt + 2, buf, 1);
+          else if (dB) load_d(5 + 2 * buf);
+        }
+        QUAD_FENCE
       }
-      QUAD_FENCE
     }
   };
-  auto first_reads = [&](int buf, V (&b)[FJ][4]) {
+  auto first_reads = [&](int buf, V (&b)[FJ][2]) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) read_b(b, ks, buf, 0);
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int j = 0; j < FJ; ++j) read_b(b, ks, j, buf, 0);
     QUAD_FENCE
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) read_a(a, ks, buf, 0);
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < FI; ++i) read_a(a, ks, i, buf, 0);
   };
 
   // Stage kt sits in buffer (kt + n_stages) & 1, so that the last two stages
@@ -1205,8 +1233,13 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
   stage(I1{}, I2{}, n_stages - 1, by, bx);
 #undef QUAD_FENCE
 #undef QUAD_SYNC
-  tile_epilogue<T, OUT_T, MODE, CFG, ADD>(g, acc, bidx, m0, n0, wave, lane, skip1x, skipx1, diag_tile,
-                                          smem);
+  tile_epilogue<T, OUT_T, MODE, CFG, ADD>(g, acc, bidx, m0, n0, wave, lane, !whole && skip1x,
+                                          !whole && skipx1, !whole && diag_tile, smem);
+  };
+  if (skip1x || skipx1 || diag_tile)
+    run(std::false_type{});
+  else
+    run(std::true_type{});
 #endif
 }
 
@@ -1220,7 +1253,7 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
 // tiles: 1024^3 symmetric with addend 12.1 / 8.7, 512^3 9.1 / 6.6, 256^3 7.4 / 5.9
 // (an empty kernel takes 4.7); a 1 x 1024x1024 Newton-Schulz call 249 / 147.
 struct SmallTile {
-  static constexpr int WM = 2, WN = 2, FI = 1, FJ = 1, waves = 4, threads = 256;
+  static constexpr int WM = 2, WN = 2, FI = 2, FJ = 2, waves = 4, threads = 256;
   static constexpr int BM = 64, BN = 64, depth = 64;
   [[maybe_unused]] static constexpr int HM = 64, HN = 64, halves = 1;
   static constexpr int stages = 8, operand = 64 * depth;  // ring depth, elements of an operand's stage
@@ -1276,7 +1309,7 @@ __device__ __forceinline__ void small_tile(const GemmArgs& g, int w) {
     const int row = pos >> 3, ch = (pos & 7) ^ ((row >> 1) & 7);
     a_off[j] = (uint32_t)min(row, g.m - 1 - m0) * (uint32_t)(2 * g.lda) + 16 * ch;
     if (BKN) {
-      const int c = (pos & 7) ^ (4 * ((row >> 1) & 1));  // row: the k-row
+      const int c = (pos & 7) ^ kn_swz<BN>(row);  // row: the k-row
       b_off[j] = (uint32_t)row * (uint32_t)(2 * g.ldb) + 2 * (uint32_t)min(c * 8, g.n - 8 - n0);
     } else {
       b_off[j] = (uint32_t)min(row, g.n - 1 - n0) * (uint32_t)(2 * g.ldb) + 16 * ch;
@@ -1303,51 +1336,55 @@ __device__ __forceinline__ void small_tile(const GemmArgs& g, int w) {
   unsigned char* tile = smem + CFG::ring_bytes;
   if (ADD) {
     const T* D = reinterpret_cast<const T*>(g.d) + bidx * g.sd + (int64_t)m0 * g.ldd + n0;
-    const uint32_t d_bytes = (uint32_t)(2 * ((g.m_lim - 1 - m0) * g.ldd + g.n_lim - n0));
+    const uint32_t d_bytes = (uint32_t)(2 * ((g.m - 1 - m0) * g.ldd + g.n - n0));
     const auto d_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)D, 0, d_bytes, 0x00020000);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int pos = (j * 4 + wave) * 64 + lane, row = pos >> 3;
       const int c = ((pos & 7) ^ epi_swz<BN>(row)) * 8;
-      const uint32_t off = (uint32_t)min(row, g.m_lim - 1 - m0) * (uint32_t)(2 * g.ldd) +
-                           2 * (uint32_t)min(c, g.n_lim - 8 - n0);
+      const uint32_t off = (uint32_t)min(row, g.m - 1 - m0) * (uint32_t)(2 * g.ldd) +
+                           2 * (uint32_t)min(c, g.n - 8 - n0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           d_rsrc, (lds_ptr_t)(reinterpret_cast<T*>(tile) + (j * 4 + wave) * 512), 16, off, 0, 0, 0);
     }
   }
 
-  const int lrow = lane & 31, lk = lane >> 5, sw = (lrow >> 1) & 7;
-  int a_rd[4], b_rd[4];  // element offsets in a stage, per k-step
+  const int G = lane >> 4, i16 = lane & 15, sw = (i16 >> 1) & 7;
+  int a_rd[2], b_rd[2], b_kn[2];  // element offsets in a stage: per k-step, per k-step, per fragment
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    a_rd[ks] = (wm * 32 + lrow) * DEPTH + (((2 * ks + lk) ^ sw) << 3);
-    b_rd[ks] = CFG::operand + (wn * 32 + lrow) * DEPTH + (((2 * ks + lk) ^ sw) << 3);
+  for (int q = 0; q < 2; ++q) {
+    a_rd[q] = (wm * 32 + i16) * DEPTH + (((4 * q + G) ^ sw) << 3);
+    b_rd[q] = CFG::operand + (wn * 32 + i16) * DEPTH + (((4 * q + G) ^ sw) << 3);
+    const int col = wn * 32 + q * 16 + 4 * (i16 & 3), kr = 8 * G + (i16 >> 2);
+    b_kn[q] = CFG::operand + kr * BN + (((col >> 3) ^ kn_swz<BN>(kr)) << 3) + (col & 7);
   }
-  const int G = lane >> 4, i16 = lane & 15, kr = i16 >> 2;
-  const int kn_col = wn * 32 + 16 * (G & 1) + 4 * (i16 & 3);
-  const int b_kn = CFG::operand + (8 * (G >> 1) + kr) * BN +
-                   (((kn_col >> 3) ^ (4 * (kr >> 1))) << 3) + (kn_col & 7);
   struct Frags {
-    V a[4], b[4];
+    V a[2][2], b[2][2];  // [fragment][k-step]
   };
   auto read = [&](Frags& f, int kt) {
     const T* stage = lds + (kt % S) * (2 * CFG::operand);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      f.a[ks] = *reinterpret_cast<const V*>(stage + a_rd[ks]);
-      if (BKN) {
-        const T* p = stage + b_kn + ks * 16 * BN;
-        v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p));
-        v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p + 4 * BN));
-        f.b[ks] = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-      } else {
-        f.b[ks] = *reinterpret_cast<const V*>(stage + b_rd[ks]);
-      }
-    }
-  };
-  f32x16 acc[1][1];
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-  for (int e = 0; e < 16; ++e) acc[0][0][e] = 0.f;
+      for (int i = 0; i < 2; ++i) {
+        f.a[i][ks] = *reinterpret_cast<const V*>(stage + a_rd[ks] + i * 16 * DEPTH);
+        if (BKN) {
+          const T* p = stage + b_kn[i] + ks * 32 * BN;
+          v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p));
+          v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p + 4 * BN));
+          f.b[i][ks] = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        } else {
+          f.b[i][ks] = *reinterpret_cast<const V*>(stage + b_rd[ks] + i * 16 * DEPTH);
+        }
+      }
+  };
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
   // Stage kt is multiplied while stage kt + 1 is read and stage kt - 1 + S requested
   // (into the slot of kt - 1, which every wave has multiplied).
   auto step = [&](auto more_, int kt, Frags& now, Frags& next) {
@@ -1361,7 +1398,12 @@ __device__ __forceinline__ void small_tile(const GemmArgs& g, int w) {
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) acc[0][0] = Mfma<T>::run(now.b[ks], now.a[ks], acc[0][0]);
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = Mfma<T>::run16(now.b[j][ks], now.a[i][ks], acc[i][j]);
   };
 #pragma unroll 1
   for (int s = 0; s < min(S - 1, n_stages); ++s) issue(s);
@@ -1753,8 +1795,8 @@ bool tiles_ok(const Problem& p) {
   constexpr int64_t kReach = (int64_t)1 << 31;
   auto reach = [](int64_t rows, int64_t ld) { return 2 * rows * ld < kReach; };
   return g.k % 64 == 0 && (g.k >= 128 || best_tile(p) == kSmall) && reach(g.m, g.lda) && reach(g.b_kn ? g.k : g.n, g.ldb) &&
-         (!g.d || (g.ldd % 8 == 0 && g.sd % 8 == 0 && g.n_lim % 8 == 0 && aligned16(g.d) &&
-                   reach(g.m_lim, g.ldd)));
+         (!g.d || (g.ldd % 8 == 0 && g.sd % 8 == 0 && g.n % 8 == 0 && aligned16(g.d) &&
+                   reach(g.m, g.ldd)));
 }
 
 // One launch of up to kMaxGroup products on one tile configuration, longest k
