@@ -553,6 +553,15 @@ __device__ __forceinline__ void wait_vm() {
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16* lds_v4i16_t;
 
+// A transpose read (ds_read_b64_tr_b16). Inlining the restrict argument gives the read
+// alias information; without it the compiler takes every direct-to-LDS load in flight
+// for a possible writer of what is read and waits for all of them (vmcnt(0)) first. The
+// kernels' own waits order the two. Measured on P X of 64 x 1408 x 2048 blocks: 616 us
+// with that wait, 467 without.
+__device__ __forceinline__ v4i16 read_transposed(lds_v4i16_t __restrict__ p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(p);
+}
+
 // One output tile: logical tile w of the problem (batch index w / tiles).
 // BKN: B is [k, n] (row-major along n, such as the iterate X of Q X) instead
 // of [n, k]. Its stages are then k-major in LDS, [k][n], with 16-byte chunk ch
@@ -884,9 +893,9 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) {
           const int ch2 = (c0 + (b + i) * CSTEP) / 8 + ((i16 & 3) >> 1);
-          const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          const v4i16 lo = read_transposed(
               (lds_v4i16_t)(tile + epi_off<BN>(row, ch2) + 4 * (i16 & 1)));
-          const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          const v4i16 hi = read_transposed(
               (lds_v4i16_t)(tile + epi_off<BN>(row + 4, ch2) + 4 * (i16 & 1)));
           v[i] = __builtin_bit_cast(u4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         }
@@ -926,9 +935,9 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
     for (int it = wave; it < (BM / 32) * (BN / 16); it += CFG::waves) {
       const int r8 = 32 * (it % (BM / 32)) + 8 * G, cc = it / (BM / 32);
       const int row = r8 + (i16 >> 2), ch = 2 * cc + ((i16 & 3) >> 1);
-      const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      const v4i16 lo = read_transposed(
           (lds_v4i16_t)(tile + epi_off<BN>(row, ch) + 4 * (i16 & 1)));
-      const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      const v4i16 hi = read_transposed(
           (lds_v4i16_t)(tile + epi_off<BN>(row + 4, ch) + 4 * (i16 & 1)));
       const int c = 16 * cc + i16;
       const int gr = m0 + r8, gc = n0 + c;
@@ -1075,8 +1084,8 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
   auto read_b = [&](V (&f)[FJ][2], int ks, int j, int buf, int h) {
     if (BKN) {
       const T* p = b_kn[j] + (2 * buf + h) * CFG::b_half + ks * 32 * HN;
-      v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p));
-      v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p + 4 * HN));
+      v4i16 lo = read_transposed((lds_v4i16_t)(p));
+      v4i16 hi = read_transposed((lds_v4i16_t)(p + 4 * HN));
       f[j][ks] = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     } else {
       f[j][ks] = *reinterpret_cast<const V*>(b_rd[ks] + (2 * buf + h) * CFG::b_half + j * 16 * DEPTH);
@@ -1370,8 +1379,8 @@ __device__ __forceinline__ void small_tile(const GemmArgs& g, int w) {
         f.a[i][ks] = *reinterpret_cast<const V*>(stage + a_rd[ks] + i * 16 * DEPTH);
         if (BKN) {
           const T* p = stage + b_kn[i] + ks * 32 * BN;
-          v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p));
-          v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t)(p + 4 * BN));
+          v4i16 lo = read_transposed((lds_v4i16_t)(p));
+          v4i16 hi = read_transposed((lds_v4i16_t)(p + 4 * BN));
           f.b[i][ks] = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         } else {
           f.b[i][ks] = *reinterpret_cast<const V*>(stage + b_rd[ks] + i * 16 * DEPTH);
