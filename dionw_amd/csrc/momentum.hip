@@ -19,9 +19,10 @@
 //               iteration reads (_matrix_step.py:172-178 and _gram.py:83-87
 //               fused), in 64 x 64 tiles (through LDS for the transpose).
 //
-// Row reductions use one 256-thread workgroup per row (its four waves sweep
+// Row reductions use one 256-thread workgroup per row, or a wave per short row with
+// the same sums (accumulate_short_kernel); a workgroup's four waves sweep
 // 4 KiB of each stream per step: 8% more HBM throughput than a wave per row at
-// 4096 columns). Thread t accumulates four partial sums (one per float4
+// 4096 columns. Thread t accumulates four partial sums (one per float4
 // component) over its float4 chunks t, t + 256, ... in column order, combines
 // them as (x + y) + (z + w); each wave combines its lanes by the xor butterfly
 // of wave_sum and the four wave sums combine as (w0 + w1) + (w2 + w3): the l1
@@ -168,6 +169,68 @@ __global__ __launch_bounds__(kRowThreads) void accumulate_kernel(AccArgs a) {
   } else if (tid == 0) {
     a.rowsq[row] = sqs;
   }
+}
+
+// The same sums, bit for bit, for rows of at most kShortCols columns: one wave per row,
+// whose lane takes the one chunk of each of the threads lane, lane + 64, + 128, + 192 of
+// accumulate_kernel's workgroup, all loaded together. A workgroup per such a row leaves
+// threads without a chunk and is mostly its launch and its reduction.
+constexpr int kShortCols = 4 * kRowThreads;
+
+template <int MODE, typename IN = float>
+__global__ __launch_bounds__(256) void accumulate_short_kernel(AccArgs a, int64_t rows) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int tensor = (int)(row / a.rows_per_tensor);
+  const int64_t local = row - (int64_t)tensor * a.rows_per_tensor;
+  const IN* g = reinterpret_cast<const IN*>(a.t.grad[tensor]) + local * a.cols;
+  f32x4* m4 = a.momentum ? reinterpret_cast<f32x4*>(a.momentum + row * a.cols) : nullptr;
+  const int n4 = (int)(a.cols >> 2);
+  f32x4 gv[4], mv[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    gv[v] = mv[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int c = lane + 64 * v;
+    if (c < n4) {
+      gv[v] = load4_nt(g, c);
+      if (m4) mv[v] = MODE == kScores ? __builtin_nontemporal_load(m4 + c) : m4[c];
+    }
+  }
+  float l1[4], sq[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int c = lane + 64 * v;
+    const f32x4 s = mv[v] + gv[v];
+    if (MODE == kScores && c < n4) __builtin_nontemporal_store(s, m4 + c);
+    f32x4 u = s;
+    if (MODE == kFullSumsq && a.nesterov) u = gv[v] + s * a.mu;
+    if (a.round_bf16) u = bf16_round4(u);
+    const f32x4 q = u * u;
+    sq[v] = wave_sum((q.x + q.y) + (q.z + q.w));
+    if (MODE == kScores) {
+      const f32x4 b = __builtin_elementwise_abs(s);
+      l1[v] = wave_sum((b.x + b.y) + (b.z + b.w));
+    }
+  }
+  if (lane != 0) return;
+  a.rowsq[row] = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+  if (MODE == kScores) a.scores[row] = (l1[0] + l1[1]) + (l1[2] + l1[3]);
+}
+
+// One launch of the row sums over `rows` rows; short vectorized rows take a wave each.
+// Measured, a workgroup / a wave per row, us: sums of squares alone 28 x 1152x576 25.8 /
+// 15.7, 64 x 4096x1024 209 / 153, 48 x 1024x256 34.7 / 18.1 (3.2 TB/s); with momentum
+// 27.8 / 23.5, 343 / 314, 36.9 / 21.4. The pass that writes momentum gains at 256 columns
+// (47 / 30) and is level or 4% slower at 576 to 1024, so it takes a wave up to 512.
+template <int MODE, typename IN = float>
+void launch_accumulate(const AccArgs& a, int64_t rows, hipStream_t stream) {
+  if (a.vec && a.cols <= (MODE == kScores ? kShortCols / 2 : kShortCols))
+    hipLaunchKernelGGL((accumulate_short_kernel<MODE, IN>), dim3((unsigned)ceil_div(rows, 4)),
+                       dim3(256), 0, stream, a, rows);
+  else
+    hipLaunchKernelGGL((accumulate_kernel<MODE, IN>), dim3((unsigned)rows), dim3(kRowThreads), 0,
+                       stream, a);
 }
 
 // den[b] = norm_denom(sum of rowsq over the block's rows); one wave per block.
@@ -486,8 +549,7 @@ int dionw_accumulate_scores(const float* const* grads, int32_t count, int64_t ro
     const int64_t rows = (int64_t)a.t.count * rows_per_tensor;
     DIONW_REQUIRE(rows * kRowThreads <= (int64_t)UINT32_MAX,
                   "accumulate_scores: %lld rows exceed one launch", (long long)rows);
-    hipLaunchKernelGGL(accumulate_kernel<kScores>, dim3((unsigned)rows), dim3(kRowThreads), 0,
-                       stream, a);
+    launch_accumulate<kScores>(a, rows, stream);
     DIONW_TRY(check_launch("accumulate_scores"));
   }
   return kOk;
@@ -518,8 +580,7 @@ int dionw_full_sumsq(const float* const* grads, int32_t count, int64_t rows_per_
     const int64_t rows = (int64_t)a.t.count * rows_per_tensor;
     DIONW_REQUIRE(rows * kRowThreads <= (int64_t)UINT32_MAX,
                   "full_sumsq: %lld rows exceed one launch", (long long)rows);
-    hipLaunchKernelGGL(accumulate_kernel<kFullSumsq>, dim3((unsigned)rows), dim3(kRowThreads), 0,
-                       stream, a);
+    launch_accumulate<kFullSumsq>(a, rows, stream);
     DIONW_TRY(check_launch("full_sumsq"));
   }
   return kOk;
@@ -565,16 +626,12 @@ int dionw_normalize_input(const void* x, int32_t x_elem, int64_t blocks, int64_t
   acc.cols = cols;
   acc.vec = vec;
   acc.round_bf16 = elem == kBF16;
-  const dim3 row_grid((unsigned)(blocks * rows));
   if (x_elem == kF32)
-    hipLaunchKernelGGL((accumulate_kernel<kFullSumsq, float>), row_grid, dim3(kRowThreads), 0,
-                       stream, acc);
+    launch_accumulate<kFullSumsq, float>(acc, blocks * rows, stream);
   else if (x_elem == kF16)
-    hipLaunchKernelGGL((accumulate_kernel<kFullSumsq, _Float16>), row_grid, dim3(kRowThreads), 0,
-                       stream, acc);
+    launch_accumulate<kFullSumsq, _Float16>(acc, blocks * rows, stream);
   else
-    hipLaunchKernelGGL((accumulate_kernel<kFullSumsq, __bf16>), row_grid, dim3(kRowThreads), 0,
-                       stream, acc);
+    launch_accumulate<kFullSumsq, __bf16>(acc, blocks * rows, stream);
   DIONW_TRY(check_launch("normalize_input"));
   hipLaunchKernelGGL(block_denom_kernel, dim3((unsigned)blocks), dim3(64), 0, stream, row_sumsq,
                      den, rows, safety, eps, (int)(elem == kBF16));
