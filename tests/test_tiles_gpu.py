@@ -74,6 +74,7 @@ def test_product_at_tile_edges(batch, m, n, k, addend, pad, dtype) -> None:
 @pytest.mark.parametrize(("batch", "n", "k", "addend"), [
     (1, 64, 128, True), (1, 64, 64, True), (2, 136, 192, True), (1, 200, 256, False), (3, 384, 384, True),
     (40, 264, 128, False), (40, 512, 512, True), (40, 392, 448, True),
+    (2, 640, 128, True), (1, 1090, 128, False), (8, 1300, 128, True),  # several column strips
 ])
 def test_symmetric_product_at_tile_edges(batch, n, k, addend) -> None:
     """A symmetric product against the full one, bit for bit above the diagonal,
