@@ -366,21 +366,16 @@ struct PipeCfg {
   static constexpr int loads_b = BN * BK / 8 / threads;
   static constexpr size_t lds_bytes = (size_t)STAGES * stage_elems * 2;
   static_assert(loads_a >= 1 && loads_b >= 1, "tile too small for the thread count");
-  static_assert(BK == 32 || BK == 64, "stage depth 32 or 64");
+  static_assert(BK == 32, "the LDS swizzle is for 32-deep stages");
 };
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-// A stage row holds BK/8 chunks of 16 bytes. Chunk q of row r sits at
-// q ^ ((r >> 2) & 3) (BK 32) or q ^ ((r >> 1) & 7) (BK 64): the 16 lanes of a
-// read phase (rows r..r+15, same chunk) cover all 64 banks once.
-template <int BK>
-__device__ __forceinline__ int swz(int row, int chunk) {
-  return BK == 32 ? chunk ^ ((row >> 2) & 3) : chunk ^ ((row >> 1) & 7);
-}
-template <int BK>
+// A stage row holds 4 chunks of 16 bytes. Chunk q of row r sits at q ^ ((r >> 2) & 3):
+// the 16 lanes of a read phase (rows r..r+15, same chunk) cover all 64 banks once.
+__device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 2) & 3); }
 __device__ __forceinline__ int plds_off(int row, int chunk) {
-  return row * BK + (swz<BK>(row, chunk) << 3);
+  return row * 32 + (swz(row, chunk) << 3);
 }
 
 // ---- LDS-staged epilogue of the large-tile kernels ------------------------------
@@ -637,7 +632,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
 #pragma unroll
   for (int j = 0; j < LA; ++j) {
     const int pos = (wave * LA + j) * 64 + lane;  // 16-byte chunk index
-    const int row = pos / CPR, logical = swz<SBK>(row, pos % CPR);
+    const int row = pos / CPR, logical = swz(row, pos % CPR);
     a_src[j] = A + (int64_t)min(m0 + row, g.m - 1) * g.lda + logical * 8;
   }
   constexpr int NCH = PBN / 8;  // 16-byte chunks per k-row of a k-major B stage
@@ -649,7 +644,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
       const int krow = pos / NCH, ch = (pos % NCH) ^ (4 * (krow % 4));
       b_src[j] = B + (int64_t)krow * g.ldb + min(n0 + ch * 8, g.n - 8);
     } else {
-      const int row = pos / CPR, logical = swz<SBK>(row, pos % CPR);
+      const int row = pos / CPR, logical = swz(row, pos % CPR);
       b_src[j] = B + (int64_t)min(n0 + row, g.n - 1) * g.ldb + logical * 8;
     }
   }
@@ -714,7 +709,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
     auto frag = [&](int ks, int set) {
 #pragma unroll
       for (int i = 0; i < FM; ++i)
-        af[set][i] = *reinterpret_cast<const V*>(As + plds_off<SBK>(wm * WTM + i * 32 + lrow, 2 * ks + lk));
+        af[set][i] = *reinterpret_cast<const V*>(As + plds_off(wm * WTM + i * 32 + lrow, 2 * ks + lk));
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         if (BKN) {
@@ -731,7 +726,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
           bfr[set][j] = __builtin_bit_cast(
               V, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
         } else {
-          bfr[set][j] = *reinterpret_cast<const V*>(Bs + plds_off<SBK>(wn * WTN + j * 32 + lrow, 2 * ks + lk));
+          bfr[set][j] = *reinterpret_cast<const V*>(Bs + plds_off(wn * WTN + j * 32 + lrow, 2 * ks + lk));
         }
       }
     };
