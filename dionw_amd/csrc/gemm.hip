@@ -1806,10 +1806,11 @@ bool tile_fits(int tile, int64_t wgs) { return tile != kSmall || wgs <= 256; }
 
 // A product's time on a tile: rounds of one workgroup per CU. Measured on 256x256 /
 // 128x128 / 64x64 tiles, us per launch of a chain: 16 x 1024^3 symmetric with addend
-// 32 / 35 / -, 36 x 768^3 31 / 40 / -, 64 x 1408 x 1408 x 2048 324 / 347 / -,
-// 16 x 1024 x 4096 x 1024 149 / 187 / -; 3584^3 69 / 59 / 128, 28 x 576^3 23 / 17 /
-// 29, 128 x 384^3 36 / 28 / 51, 4 x 1024^3 27 / 15 / 22; 1024^3 26 / 14 / 9,
-// 12 x 384^3 18 / 10 / 7, 256^3 16 / 9 / 6 (64 x 64 x 64: 6; an empty kernel: 4.7).
+// 30 / 31 / 63, 36 x 768^3 29 / 30 / 66, 64 x 1408 x 1408 x 2048 296 / 315 / 697,
+// 16 x 1024 x 4096 x 1024 127 / 175 / 401; 3584^3 68 / 52 / 128, 28 x 576^3 21 / 16 /
+// 28, 128 x 384^3 33 / 24 / 49, 4 x 1024^3 27 / 14 / 22, 8 x 512^3 19 / 10 / 12;
+// 1024^3 26 / 13 / 9, 12 x 384^3 17 / 9 / 6.5, 256^3 13 / 8 / 6 (64 x 64 x 64: 6; an
+// empty kernel: 4.7). The rule takes the fastest on all of them.
 double product_time(const Problem& p, int tile) {
   const int64_t wgs = wgs_of(p, kTileSide[tile]);
   if (!tile_fits(tile, wgs)) return 1e300;
