@@ -1135,9 +1135,13 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
 
   V a[FI][2], bx[FJ][2], by[FJ][2];
 #define QUAD_FENCE __builtin_amdgcn_sched_barrier(0);
-#define QUAD_SYNC(VM)                                                           \
+  // READS: the wave's last LDS reads that may still be on their way when it meets the
+  // others; the slots refilled after the sync must not be among theirs. Reads are waited
+  // for by the MFMAs that use them, but a quadrant that is not multiplied uses none, so
+  // every count here has to hold with any of the quadrants left out.
+#define QUAD_SYNC(VM, READS)                                                    \
   QUAD_FENCE                                                                    \
-  wait_vm<VM, 2 * FI>();                                                        \
+  wait_vm<VM, READS>();                                                         \
   __builtin_amdgcn_s_barrier();                                                 \
   QUAD_FENCE
   // One row fragment of a quadrant over 32 k; the MFMA takes B first, so that a
@@ -1159,8 +1163,9 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
     constexpr int buf = decltype(buf_)::value, tail = decltype(tail_)::value;
     constexpr int dA = ADD ? L : 0, dB = D_SLOTS == 8 ? dA : 0;
     static_assert(FI >= FJ, "a row fragment's step for every column fragment's read");
-    // rows half 0 x columns half 0; B1(kt) is read
-    QUAD_SYNC((tail != 2 ? 3 * L : dA + 2 * dB))
+    // rows half 0 x columns half 0; B1(kt) is read. Pending: A0(kt). Refilled next:
+    // A1(kt - 1), B0(kt), both read before it.
+    QUAD_SYNC((tail != 2 ? 3 * L : dA + 2 * dB), 2 * FI)
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
@@ -1188,9 +1193,9 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
         QUAD_FENCE
       }
     }
-    // 1 x 1; B0(kt + 1) replaces B1(kt)
+    // 1 x 1; B0(kt + 1) replaces B1(kt). Pending: A1(kt). Refilled next: A0(kt), B1(kt).
     if (tail != 2 || ADD) {
-      QUAD_SYNC((tail == 0 ? 3 * L : tail == 1 ? 2 * L + dB : 63))
+      QUAD_SYNC((tail == 0 ? 3 * L : tail == 1 ? 2 * L + dB : 63), 2 * FI)
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -1211,7 +1216,9 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
     }
     // 1 x 0; A0(kt + 1) replaces A1(kt)
     if (tail == 2 && ADD) {
-      QUAD_SYNC(63)
+      // A1(kt) itself is refilled, and no read followed its own: none may be pending
+      // (without 1 x 1, nothing has waited for them).
+      QUAD_SYNC(63, 0)
       load_d(2 * buf + 1);
     }
 #pragma unroll
@@ -1250,7 +1257,7 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
   load_b(1, p0 ^ 1, 0);
   load_a(1, p0 ^ 1, 0);
   load_b(1, p0 ^ 1, 1);
-  QUAD_SYNC((5 * L))
+  QUAD_SYNC((5 * L), 2 * FI)
   int kt = 0;
   if (p0) {
     first_reads(1, by);

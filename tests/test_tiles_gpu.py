@@ -111,3 +111,25 @@ def test_left_products_read_the_iterate_as_it_lies(blocks: int, r: int, c: int) 
         y = 3.4445 * y + torch.matmul(2.0315 * torch.matmul(gram, gram) - 4.7750 * gram, y)
     for b in range(blocks):
         assert (got[b] - y[b]).norm() <= 0.03 * y[b].norm(), f"block {b}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("k", [128, 192, 448])
+@pytest.mark.parametrize(("batch", "m", "n"), [
+    (40, 512, 640),  # 256x256 tiles, the last column's half empty
+    (40, 256, 192),  # 128x128 tiles, the same
+])
+def test_addend_in_tiles_without_a_right_half(batch, m, n, k, dtype) -> None:
+    """The addend's last rows go to the slot of the row operand's second half while
+    that half is still to be multiplied: against float64, and the same bits again."""
+    print(f"{batch} x {m}x{n}x{k} {dtype}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a, b, d = (_strided(shape, 0, dtype, g)
+               for shape in ((batch, m, k), (batch, n, k), (batch, m, n)))
+    got = gemm_nt(a, b, d=d, alpha=0.5, beta=-1.25)
+    product = 0.5 * torch.matmul(a.double(), b.double().mT.contiguous()) - 1.25 * d.double()
+    scale = (0.5 * torch.matmul(a.double().abs(), b.double().abs().mT.contiguous())
+             + 1.25 * d.double().abs())
+    _check(got, product, scale, k, "out")
+    for _ in range(3):
+        assert torch.equal(gemm_nt(a, b, d=d, alpha=0.5, beta=-1.25), got)
