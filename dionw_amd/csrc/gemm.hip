@@ -2,8 +2,9 @@
 //
 // Every product is one "NT" form, C[i,j] = sum_k A[i,k] B[j,k] with both
 // operands row-major along k, computed with v_mfma_f32_16x16x32_{f16,bf16} from
-// 64-deep LDS-staged k tiles, or v_mfma_f32_32x32x16_* where k is no multiple of 64
-// (fp32 accumulation, every element over k in order, whatever the tile). The epilogue forms
+// 64-deep LDS-staged k tiles, or v_mfma_f32_32x32x16_* where k is no multiple of 64 and
+// for what those tiles refuse (tiles_ok; fp32 accumulation, every element over k in
+// order, whatever the tile). The epilogue forms
 // alpha * acc + beta * D[i,j] and rounds once to the storage type; in mode
 // kOutRoundAcc it rounds the product to the storage type first, then forms
 // alpha * bf16(acc) + beta * D and rounds again (a product stored by one
@@ -343,13 +344,17 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_nt_kernel(GemmArgs g) {
 
 // ---- pipelined tile kernels ----------------------------------------------------
 //
-// For the products that the quadrant tiles below do not take (depths that are an
-// odd multiple of 32, or 64; an addend whose rows are not 16-byte chunks; operands
-// past 2 GB): 256x256 per workgroup of 16 waves (4x4, 64x64 per wave) or 128x128
-// per workgroup of 4 waves (2x2, two workgroups per CU). k advances through an LDS
-// ring of four 32-deep stages filled by direct-to-LDS loads, a stage requested
-// three stages before it is consumed. Waits are explicit: before a stage is read
-// every wave waits for its own loads of it (vmcnt) and for its reads of the stage
+// For the products that the 64-deep tiles below do not take (depths that are an odd
+// multiple of 32; a depth of 64 on many tiles; an addend whose rows are not 16-byte
+// chunks; operands past 2 GB): 256x256 per workgroup of 16 waves (4x4, 64x64 per
+// wave) or 128x128 per workgroup of 4 waves (2x2, two workgroups per CU). k advances
+// through an LDS ring filled by direct-to-LDS loads: two 64-deep stages where k is a
+// multiple of 64, else four 32-deep ones; a stage is requested one stage (64-deep) or
+// three stages (32-deep) before it is consumed. On 32-deep stages the multiples of 64
+// take 4 to 17% longer (us, 64-deep / 32-deep: 36 x 768^3 with an addend in rows of
+// 772 101 / 118, 8 x 3584^3 in rows of 3588 971 / 1031, 65600 x 1024 x 16384 2155 /
+// 2330, 64 x 513 x 248 x 64 with addend 17 / 20). Waits are explicit: before a stage is
+// read every wave waits for its own loads of it (vmcnt) and for its reads of the stage
 // about to be refilled (lgkmcnt), then the workgroup meets at one barrier. Rows
 // beyond m / n load a clamped valid row (only outputs that are never stored see
 // them), so every wave issues the same number of loads per stage and the vmcnt
@@ -366,16 +371,21 @@ struct PipeCfg {
   static constexpr int loads_b = BN * BK / 8 / threads;
   static constexpr size_t lds_bytes = (size_t)STAGES * stage_elems * 2;
   static_assert(loads_a >= 1 && loads_b >= 1, "tile too small for the thread count");
-  static_assert(BK == 32, "the LDS swizzle is for 32-deep stages");
+  static_assert(BK == 32 || BK == 64, "stage depth 32 or 64");
 };
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-// A stage row holds 4 chunks of 16 bytes. Chunk q of row r sits at q ^ ((r >> 2) & 3):
-// the 16 lanes of a read phase (rows r..r+15, same chunk) cover all 64 banks once.
-__device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 2) & 3); }
+// A stage row holds BK/8 chunks of 16 bytes. Chunk q of row r sits at
+// q ^ ((r >> 2) & 3) (BK 32) or q ^ ((r >> 1) & 7) (BK 64): the 16 lanes of a
+// read phase (rows r..r+15, same chunk) cover all 64 banks once.
+template <int BK>
+__device__ __forceinline__ int swz(int row, int chunk) {
+  return BK == 32 ? chunk ^ ((row >> 2) & 3) : chunk ^ ((row >> 1) & 7);
+}
+template <int BK>
 __device__ __forceinline__ int plds_off(int row, int chunk) {
-  return row * 32 + (swz(row, chunk) << 3);
+  return row * BK + (swz<BK>(row, chunk) << 3);
 }
 
 // ---- LDS-staged epilogue of the large-tile kernels ------------------------------
@@ -632,7 +642,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
 #pragma unroll
   for (int j = 0; j < LA; ++j) {
     const int pos = (wave * LA + j) * 64 + lane;  // 16-byte chunk index
-    const int row = pos / CPR, logical = swz(row, pos % CPR);
+    const int row = pos / CPR, logical = swz<SBK>(row, pos % CPR);
     a_src[j] = A + (int64_t)min(m0 + row, g.m - 1) * g.lda + logical * 8;
   }
   constexpr int NCH = PBN / 8;  // 16-byte chunks per k-row of a k-major B stage
@@ -644,7 +654,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
       const int krow = pos / NCH, ch = (pos % NCH) ^ (4 * (krow % 4));
       b_src[j] = B + (int64_t)krow * g.ldb + min(n0 + ch * 8, g.n - 8);
     } else {
-      const int row = pos / CPR, logical = swz(row, pos % CPR);
+      const int row = pos / CPR, logical = swz<SBK>(row, pos % CPR);
       b_src[j] = B + (int64_t)min(n0 + row, g.n - 1) * g.ldb + logical * 8;
     }
   }
@@ -709,7 +719,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
     auto frag = [&](int ks, int set) {
 #pragma unroll
       for (int i = 0; i < FM; ++i)
-        af[set][i] = *reinterpret_cast<const V*>(As + plds_off(wm * WTM + i * 32 + lrow, 2 * ks + lk));
+        af[set][i] = *reinterpret_cast<const V*>(As + plds_off<SBK>(wm * WTM + i * 32 + lrow, 2 * ks + lk));
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         if (BKN) {
@@ -726,7 +736,7 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, int w) {
           bfr[set][j] = __builtin_bit_cast(
               V, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
         } else {
-          bfr[set][j] = *reinterpret_cast<const V*>(Bs + plds_off(wn * WTN + j * 32 + lrow, 2 * ks + lk));
+          bfr[set][j] = *reinterpret_cast<const V*>(Bs + plds_off<SBK>(wn * WTN + j * 32 + lrow, 2 * ks + lk));
         }
       }
     };
@@ -1889,8 +1899,10 @@ int launch_group_typed(const std::vector<const Problem*>& ps, int tile, hipStrea
 
 template <typename T, typename OUT_T, int MODE>
 int launch_typed(const Problem& p, hipStream_t stream) {
-  // Depths that are an odd multiple of 32 (and what tiles_ok refuses) run 32-deep
-  // stages in a ring of four.
+  // What tiles_ok refuses: 64-deep stages in a ring of two, or 32-deep ones in a ring
+  // of four where the depth is an odd multiple of 32.
+  using Big64 = PipeCfg<256, 256, 4, 4, 2, 64>;
+  using Mid64 = PipeCfg<128, 128, 2, 2, 2, 64>;
   using Big32 = PipeCfg<256, 256, 4, 4, 4, 32>;
   using Mid32 = PipeCfg<128, 128, 2, 2, 4, 32>;
   const bool k32 = p.g.k % 32 == 0;
@@ -1905,9 +1917,20 @@ int launch_typed(const Problem& p, hipStream_t stream) {
       default: return launch_tile<T, OUT_T, MODE, SmallTile>(p, stream);
     }
   }
+  if (p.g.k % 64 == 0) {
+    // Rounds of one 256x256 or two 128x128 workgroups per CU, the smaller at 0.65 of the
+    // larger's time (us, 256x256 / 128x128, rows of n + 4: 36 x 768^3 with addend 114 /
+    // 101, 64 x 1408^3 symmetric with addend 428 / 450, where the costs are 40 / 39 and
+    // 120 / 117; elsewhere the shorter one is taken).
+    const int64_t big = 20 * ((wgs_of(p, 256) + 255) / 256);
+    const int64_t mid = 13 * ((wgs_of(p, 128) + 511) / 512);
+    return big <= mid ? launch_pipe<T, OUT_T, MODE, Big64>(p, stream)
+                      : launch_pipe<T, OUT_T, MODE, Mid64>(p, stream);
+  }
   if (k32)
-    return product_time(p, kBig) <= product_time(p, kMid) ? launch_pipe<T, OUT_T, MODE, Big32>(p, stream)
-                                      : launch_pipe<T, OUT_T, MODE, Mid32>(p, stream);
+    return product_time(p, kBig) <= product_time(p, kMid)
+               ? launch_pipe<T, OUT_T, MODE, Big32>(p, stream)
+               : launch_pipe<T, OUT_T, MODE, Mid32>(p, stream);
   if (wgs_of(p, 128) >= 512) return launch_cfg<T, OUT_T, 128, 128, 2, 2, MODE>(p, stream);
   return launch_cfg<T, OUT_T, 64, 64, 2, 2, MODE>(p, stream);
 }

@@ -133,3 +133,46 @@ def test_addend_in_tiles_without_a_right_half(batch, m, n, k, dtype) -> None:
     _check(got, product, scale, k, "out")
     for _ in range(3):
         assert torch.equal(gemm_nt(a, b, d=d, alpha=0.5, beta=-1.25), got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize(("batch", "m", "n", "k", "symmetric"), [
+    (1, 130, 72, 128, False),    # 128x128 tiles of the ring of two 64-deep stages,
+    (3, 392, 385, 448, False),   # with ragged rows and columns,
+    (36, 768, 768, 192, False),
+    (36, 768, 760, 64, False),   # one stage;
+    (40, 520, 520, 320, False),  # 256x256 tiles,
+    (64, 500, 500, 64, False),   # one stage
+    (2, 264, 264, 192, True), (36, 520, 520, 128, True),
+])
+def test_addend_in_rows_that_are_no_chunks(batch, m, n, k, symmetric, dtype) -> None:
+    """An addend whose rows are not 16-byte chunks, at depths that are a multiple of 64."""
+    print(f"{batch} x {m}x{n}x{k} symmetric {symmetric} {dtype}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a = _strided((batch, m, k), 0, dtype, g)
+    b = a if symmetric else _strided((batch, n, k), 8, dtype, g)
+    d = _strided((batch, m, n), 4 if n % 2 == 0 else 3, dtype, g)
+    if symmetric:
+        d.copy_(d + d.mT)
+    got = gemm_nt(a, b, d=d, alpha=0.5, beta=-1.25, symmetric=symmetric,
+                  out=torch.empty(batch, m, n, device=DEV, dtype=dtype))
+    product = 0.5 * torch.matmul(a.double(), b.double().mT.contiguous()) - 1.25 * d.double()
+    scale = (0.5 * torch.matmul(a.double().abs(), b.double().abs().mT.contiguous())
+             + 1.25 * d.double().abs())
+    _check(got, product, scale, k, "out")
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_operand_past_2_gb(wide) -> None:
+    """Rows past the 2 GB that a tile's byte offsets reach, read and multiplied in place:
+    the first and last rows against float64."""
+    m, n, k = 65600, 136, 16384
+    print(f"{m}x{n}x{k} wide {wide}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(7)
+    long = torch.randn(m, k, device=DEV, generator=g, dtype=torch.float16)
+    short = torch.randn(n, k, device=DEV, generator=g, dtype=torch.float16)
+    got = gemm_nt(short, long) if wide else gemm_nt(long, short)
+    got = got.mT if wide else got
+    for rows in (slice(0, 64), slice(m - 200, m)):
+        a, b = long[rows].double(), short.double()
+        _check(got[rows], a @ b.T.contiguous(), a.abs() @ b.T.abs().contiguous(), k, str(rows))
