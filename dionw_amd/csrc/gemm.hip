@@ -345,7 +345,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_nt_kernel(GemmArgs g) {
 // ---- pipelined tile kernels ----------------------------------------------------
 //
 // For the products that the 64-deep tiles below do not take (depths that are an odd
-// multiple of 32; a depth of 64 on many tiles; an addend whose rows are not 16-byte
+// multiple of 32; a depth of 64 on larger tiles; an addend whose rows are not 16-byte
 // chunks; operands past 2 GB): 256x256 per workgroup of 16 waves (4x4, 64x64 per
 // wave) or 128x128 per workgroup of 4 waves (2x2, two workgroups per CU). k advances
 // through an LDS ring filled by direct-to-LDS loads: two 64-deep stages where k is a
@@ -1303,14 +1303,27 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
 // before; one barrier per stage. Measured in a chain of launches, us, against 128x128
 // tiles: 1024^3 symmetric with addend 12.1 / 8.7, 512^3 9.1 / 6.6, 256^3 7.4 / 5.9
 // (an empty kernel takes 4.7); a 1 x 1024x1024 Newton-Schulz call 249 / 147.
+// The ring has no more slots than the product has stages, so that the workgroups of a
+// one-stage product take 24 KB and share a CU: such products run these tiles whatever
+// their number. On 128x128 tiles / here, us: 1000 x 64^3 with addend 19.5 / 9.8, 3000 x
+// 64x256x64 117 / 58; Gram calls on 432 x 64x768 349 / 171, 455 x 48x192 292 / 124,
+// 16384 x 64x64 5370 / 1450. (A whole ring each takes 272 on the first of these calls.)
 struct SmallTile {
   static constexpr int WM = 2, WN = 2, FI = 2, FJ = 2, waves = 4, threads = 256;
   static constexpr int BM = 64, BN = 64, depth = 64;
   [[maybe_unused]] static constexpr int HM = 64, HN = 64, halves = 1;
   static constexpr int stages = 8, operand = 64 * depth;  // ring depth, elements of an operand's stage
-  static constexpr size_t ring_bytes = (size_t)stages * 2 * operand * 2;
-  static constexpr size_t lds_bytes = ring_bytes + (size_t)BM * BN * 2;
+  static constexpr size_t slot_bytes = (size_t)2 * operand * 2, tile_bytes = (size_t)BM * BN * 2;
+  static constexpr size_t lds_bytes = stages * slot_bytes + tile_bytes;
 };
+
+// LDS of a workgroup on a product of depth k.
+template <typename CFG>
+size_t tile_lds(int64_t k) {
+  if constexpr (std::is_same<CFG, SmallTile>::value)
+    return (size_t)std::min<int64_t>(CFG::stages, k / CFG::depth) * CFG::slot_bytes + CFG::tile_bytes;
+  return CFG::lds_bytes;
+}
 
 // s_waitcnt for at most 4 n loads in flight, n <= 6.
 __device__ __forceinline__ void wait_small(int n) {
@@ -1332,7 +1345,7 @@ __device__ __forceinline__ void small_tile(const GemmArgs& g, int w) {
   constexpr int DEPTH = CFG::depth, S = CFG::stages, BM = CFG::BM, BN = CFG::BN;
   using V = typename Mfma<T>::vec;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  T* lds = reinterpret_cast<T*>(smem);  // [stage][A 64x64, B 64x64], then the output tile
+  T* lds = reinterpret_cast<T*>(smem);  // [slot][A 64x64, B 64x64], then the output tile
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1384,7 +1397,7 @@ __device__ __forceinline__ void small_tile(const GemmArgs& g, int w) {
           kt * b_step, 0, 0);
     }
   };
-  unsigned char* tile = smem + CFG::ring_bytes;
+  unsigned char* tile = smem + min(S, n_stages) * CFG::slot_bytes;
   if (ADD) {
     const T* D = reinterpret_cast<const T*>(g.d) + bidx * g.sd + (int64_t)m0 * g.ldd + n0;
     const uint32_t d_bytes = (uint32_t)(2 * ((g.m - 1 - m0) * g.ldd + g.n - n0));
@@ -1778,14 +1791,13 @@ int launch_pipe(const Problem& p, hipStream_t stream) {
 
 template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
 int launch_tile_kn(const Problem& p, hipStream_t stream) {
-  constexpr size_t lds_bytes = CFG::lds_bytes;
   constexpr auto kern = gemm_nt_tile_kernel<T, OUT_T, MODE, CFG, BKN, ADD>;
-  DIONW_TRY(allow_lds<kern>(lds_bytes));
+  DIONW_TRY(allow_lds<kern>(CFG::lds_bytes));
   GemmArgs g;
   const int64_t wgs = pipe_args<CFG>(p, g);
   if (wgs < 0) return kInvalid;
-  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(CFG::threads), lds_bytes, stream, g,
-                     (int)p.batch);
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(CFG::threads), tile_lds<CFG>(p.g.k), stream,
+                     g, (int)p.batch);
   return check_launch("gemm_nt_tile");
 }
 
@@ -1816,10 +1828,13 @@ double tile_time(int tile, int64_t k) {
   return stage[tile] * (double)k / 64.0 + fixed[tile];
 }
 
-// Whether a tile may run `wgs` workgroups: 64x64 tiles only where one round holds
-// them all. Their ring fills a CU's LDS, so that a second round waits for the
-// first, and they read four times the operand bytes of 256x256 ones.
-bool tile_fits(int tile, int64_t wgs) { return tile != kSmall || wgs <= 256; }
+// Whether a tile may run `wgs` workgroups of depth k: 64x64 tiles only where one round
+// holds them all or the depth is one stage. A longer ring fills a CU's LDS, so that a
+// second round waits for the first, and they read four times the operand bytes of
+// 256x256 ones.
+bool tile_fits(int tile, int64_t wgs, int64_t k) {
+  return tile != kSmall || wgs <= 256 || k == SmallTile::depth;
+}
 
 // A product's time on a tile: rounds of one workgroup per CU. Measured on 256x256 /
 // 128x128 / 64x64 tiles, us per launch of a chain: 16 x 1024^3 symmetric with addend
@@ -1830,7 +1845,7 @@ bool tile_fits(int tile, int64_t wgs) { return tile != kSmall || wgs <= 256; }
 // empty kernel: 4.7). The rule takes the fastest on all of them.
 double product_time(const Problem& p, int tile) {
   const int64_t wgs = wgs_of(p, kTileSide[tile]);
-  if (!tile_fits(tile, wgs)) return 1e300;
+  if (!tile_fits(tile, wgs, p.g.k)) return 1e300;
   return (double)((wgs + 255) / 256) * tile_time(tile, p.g.k);
 }
 int best_tile(const Problem& p) {
@@ -1874,7 +1889,8 @@ int launch_tile_group_kn(const std::vector<const Problem*>& ps, hipStream_t stre
       return kInvalid;
     }
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)start), dim3(CFG::threads), CFG::lds_bytes, stream, grp);
+  hipLaunchKernelGGL(kern, dim3((unsigned)start), dim3(CFG::threads),
+                     tile_lds<CFG>(order[0]->g.k), stream, grp);
   return check_launch("gemm_nt_tile_group");
 }
 
@@ -1980,15 +1996,12 @@ int launch(const Problem& p, hipStream_t stream) {
 // (kRamp, about 6 us).
 constexpr double kRamp = 5.3;
 
-int64_t shortest_depth(const std::vector<const Problem*>& ps) {
-  int64_t k = INT64_MAX;
-  for (const Problem* p : ps) k = std::min<int64_t>(k, p->g.k);
-  return k;
-}
-
 int group_plan(const std::vector<const Problem*>& ps, bool pair) {
   double separate = 0.0, ramp = 0.0;
+  int64_t k_min = INT64_MAX, k_max = 0;
   for (const Problem* p : ps) {
+    k_min = std::min<int64_t>(k_min, p->g.k);
+    k_max = std::max<int64_t>(k_max, p->g.k);
     const int tile = best_tile(*p);
     const bool ramps = pair || wgs_of(*p, kTileSide[tile]) <= 256;
     if (ramps) ramp = kRamp;
@@ -2006,7 +2019,7 @@ int group_plan(const std::vector<const Problem*>& ps, bool pair) {
       longest = std::max(longest, one);
       shortest = std::min(shortest, one);
     }
-    if (!tile_fits(c, wgs) || (c != kSmall && shortest_depth(ps) < 128)) continue;
+    if (!tile_fits(c, wgs, k_max) || (c != kSmall && k_min < 128)) continue;
     const double total = ramp + (wgs <= 256 ? longest : std::max(longest, work + 0.5 * shortest));
     if (total < separate) {
       separate = total;

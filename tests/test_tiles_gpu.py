@@ -176,3 +176,43 @@ def test_operand_past_2_gb(wide) -> None:
     for rows in (slice(0, 64), slice(m - 200, m)):
         a, b = long[rows].double(), short.double()
         _check(got[rows], a @ b.T.contiguous(), a.abs() @ b.T.abs().contiguous(), k, str(rows))
+
+
+@pytest.mark.parametrize(("batch", "m", "n", "addend"), [
+    (257, 64, 64, True), (300, 50, 72, True), (3000, 64, 64, False), (90, 130, 88, True),
+    (40, 513, 64, True),
+])
+def test_one_stage_on_many_small_tiles(batch, m, n, addend) -> None:
+    """Depth 64 on more 64x64 tiles than CUs, whose workgroups hold one stage and share
+    a CU."""
+    print(f"{batch} x {m}x{n}x64 addend {addend}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    a = _strided((batch, m, 64), 0, torch.bfloat16, g)
+    b = _strided((batch, n, 64), 8, torch.bfloat16, g)
+    d = _strided((batch, m, n), 8, torch.bfloat16, g) if addend else None
+    out = torch.full((batch, m, n + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+    out_t = torch.full((batch, n, m + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+    gemm_nt(a, b, d=d, alpha=0.5, beta=-1.25 if addend else 0.0, out=out[:, :, :n],
+            out_t=out_t[:, :, :m])
+    product = 0.5 * torch.matmul(a.double(), b.double().mT.contiguous())
+    scale = 0.5 * torch.matmul(a.double().abs(), b.double().abs().mT.contiguous())
+    if addend:
+        product -= 1.25 * d.double()
+        scale += 1.25 * d.double().abs()
+    _check(out[:, :, :n], product, scale, 64, "out")
+    assert torch.equal(out_t[:, :, :m], out[:, :, :n].mT)
+    assert (out[:, :, n:] == 7).all() and (out_t[:, :, m:] == 7).all(), "wrote past the rows"
+
+
+@pytest.mark.parametrize("kind", [NewtonSchulz.GRAM, NewtonSchulz.KELLER, NewtonSchulz.POLAR_EXPRESS_TRITON])
+@pytest.mark.parametrize(("rows", "cols"), [(48, 192), (64, 130), (200, 60)])
+def test_many_thin_blocks_are_iterated_alike(rows: int, cols: int, kind) -> None:
+    """A block of a batch of 300 thin blocks, whose products take several rounds of
+    one-stage tiles, has the bits that it has alone."""
+    print(f"300 x {rows}x{cols} {kind}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows + cols)
+    x = torch.randn(300, rows, cols, device=DEV, generator=g)
+    f = newton_schulz_fn(kind)
+    got = f(x, 1e-8)
+    for b in (0, 7, 255, 256, 299):
+        assert torch.equal(got[b], f(x[b:b + 1], 1e-8)[0]), f"block {b}"
