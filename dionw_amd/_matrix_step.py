@@ -81,10 +81,13 @@ NEWTON_SCHULZ_EPS: Final[float] = 1e-8
 # on smaller GPUs (_matrix_step.py:40-50). The fused passes here hold no float32
 # copy: a run keeps its selected rows in fp16 (in one or both orientations), the
 # bf16 output and the Newton-Schulz workspace (six fp16 r x r matrices and one
-# r x c per block): at most 20 bytes per update element (square blocks), under
-# 22 GB at this cap (17 GB for the Llama-3-8B gate/up bucket). Bigger runs fill
-# the 256 CUs better (fewer partly idle tile rounds per product) and launch
-# fewer kernels; every Llama-3-8B bucket is one run.
+# r x c per block): at most 20 bytes per update element (square blocks, sides
+# rounded up to 8), under 22 GB at this cap (17 GB for the Llama-3-8B gate/up
+# bucket). The padding of thin blocks to whole tiles may pass 20 bytes an element
+# up to 8 GiB a run (tile_sides), and without that bound only in runs of more than
+# 65535 blocks with a side that rounds up to no multiple of 32 (under 70 bytes).
+# Bigger runs fill the 256 CUs better (fewer partly idle tile rounds per product)
+# and launch fewer kernels; every Llama-3-8B bucket is one run.
 MAX_RUN_ELEMENTS: Final[int] = 2**30
 
 

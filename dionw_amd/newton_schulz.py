@@ -59,6 +59,8 @@ def _round8(n: int) -> int:
     return (n + 7) // 8 * 8
 
 
+# The library takes short sides below this.
+_SIDE_LIMIT = 1 << 16
 # Whether an iterate whose short side is an odd multiple of 32 (at least 256)
 # is padded with zero rows to the next multiple of 64.
 PAD_SHORT_SIDE_TO_64 = True
@@ -71,13 +73,15 @@ def padded_sides(rows: int, cols: int) -> tuple[int, int]:
     depth is that side run 64-deep LDS stages (the padding rows are zero, which
     every polynomial here keeps exactly zero, and are never stored).
 
-    The short side grows only while it stays no longer than the long side: the
-    iteration runs in the orientation of the unpadded block (wide: short side
-    first), and the library needs the first padded extent to be the shorter.
+    The short side grows only while it stays no longer than the long side and below
+    the library's limit: the iteration runs in the orientation of the unpadded block
+    (wide: short side first), and the library needs the first padded extent to be the
+    shorter.
     """
     p_pad, j_pad = _round8(rows), _round8(cols)
     short, long = min(p_pad, j_pad), max(p_pad, j_pad)
-    if PAD_SHORT_SIDE_TO_64 and short >= 256 and short % 64 == 32 and short + 32 <= long:
+    if (PAD_SHORT_SIDE_TO_64 and short >= 256 and short % 64 == 32
+            and short + 32 <= min(long, _SIDE_LIMIT - 1)):
         if rows <= cols:
             p_pad += 32
         else:
@@ -85,10 +89,22 @@ def padded_sides(rows: int, cols: int) -> tuple[int, int]:
     return p_pad, j_pad
 
 
-# A batch is padded to the tiles' multiple of 64 where that at most quadruples it or
-# leaves it this small (elements of the prepared input).
 _TILE_SIDE = 64
+# A batch is padded to whole tiles where that at most quadruples the prepared input or
+# leaves it this small (its elements), ...
 _PAD_GROWTH, _PAD_ELEMENTS = 4, 1 << 24
+# ... and where the buffers of the iteration stay within what a batch of square blocks
+# takes without padding (bytes per element), or within this total.
+SCRATCH_PER_ELEMENT, PAD_SCRATCH = 20, 8 << 30
+# Products whose depth is no multiple of 32 take no more blocks than this.
+_RAGGED_BLOCKS = 65535
+
+
+def _scratch_bytes(blocks: int, rows: int, cols: int, sides: tuple[int, int]) -> int:
+    """Bytes of a batch's buffers at ``sides``: the prepared input, the output and the
+    largest workspace (the Gram iteration's six squares of the short side and one input)."""
+    r, c = min(sides), max(sides)
+    return 2 * blocks * (r * c + rows * cols + 6 * r * r + r * c)
 
 
 def tile_sides(blocks: int, rows: int, cols: int) -> tuple[int, int]:
@@ -97,16 +113,26 @@ def tile_sides(blocks: int, rows: int, cols: int) -> tuple[int, int]:
     no transposed copy (the padding is zero and stays zero); ``padded_sides`` for
     batches of so many thin blocks that the padding would dominate their memory.
 
-    Measured, three 500x1301 blocks through the cuBLAS-rounded Keller quintic: 260 us
-    at (504, 1304), whose products run the register-staged 64x64 kernel, 188 us at
-    (512, 1344); a step of six layers of side 200 with an EMA 1500 and 1170 us.
+    A batch's buffers take at most ``SCRATCH_PER_ELEMENT`` bytes per element of the
+    blocks with sides rounded up to 8, or ``PAD_SCRATCH`` in all where that is more;
+    padding past that is for batches that only the padded products can take.
+
+    Measured at sides rounded up to 8 / to 64: three 500x1301 blocks through the
+    cuBLAS-rounded Keller quintic 260 / 188 us; a step of six layers of side 200 with an
+    EMA 1500 / 1170 us; Gram calls on 4096 x 16x64 1542 / 385 us (38 / 269 MB of
+    buffers), 41943 x 40x40 18.5 / 3.2 ms (1.2 / 2.8 GB), 12945 x 72x72 8.1 / 3.6 ms
+    (1.2 / 3.4 GB), 1820 x 96x384 1.29 / 0.96 ms (0.47 / 0.72 GB), 3072 x 80x2560 6.4 /
+    4.6 ms (4.0 / 4.6 GB).
     """
     p_pad, j_pad = (-(-n // _TILE_SIDE) * _TILE_SIDE for n in (rows, cols))
+    if min(p_pad, j_pad) >= _SIDE_LIMIT:
+        return padded_sides(rows, cols)
     padded, plain = p_pad * j_pad, _round8(rows) * _round8(cols)
     small = padded <= _PAD_GROWTH * plain or blocks * padded <= _PAD_ELEMENTS
-    if small and min(p_pad, j_pad) < 1 << 16:  # the library's limit on the short side
-        return p_pad, j_pad
-    return padded_sides(rows, cols)
+    held = _scratch_bytes(blocks, rows, cols, (p_pad, j_pad)) <= max(
+        SCRATCH_PER_ELEMENT * blocks * plain, PAD_SCRATCH)
+    only = blocks > _RAGGED_BLOCKS and (_round8(rows) % 32 or _round8(cols) % 32)
+    return (p_pad, j_pad) if small and (held or only) else padded_sides(rows, cols)
 
 
 def prepared_orientations(rows: int, cols: int,
