@@ -1309,7 +1309,8 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
 // 64x256x64 117 / 58; Gram calls on 432 x 64x768 349 / 171, 455 x 48x192 292 / 124,
 // 16384 x 64x64 5370 / 1450. (A whole ring each takes 272 on the first of these calls.)
 struct SmallTile {
-  static constexpr int WM = 2, WN = 2, FI = 2, FJ = 2, waves = 4, threads = 256;
+  [[maybe_unused]] static constexpr int WM = 2, WN = 2, FI = 2, FJ = 2, waves = 4;
+  static constexpr int threads = 256;
   static constexpr int BM = 64, BN = 64, depth = 64;
   [[maybe_unused]] static constexpr int HM = 64, HN = 64, halves = 1;
   static constexpr int stages = 8, operand = 64 * depth;  // ring depth, elements of an operand's stage
@@ -1783,10 +1784,37 @@ int launch_pipe_kn(const Problem& p, hipStream_t stream) {
   return check_launch("gemm_nt_pipe");
 }
 
+int no_kernel() {
+  set_error("gemm: no kernel for this form of the output mode");
+  return kInvalid;
+}
+
+// The Gram iteration's last product is a left product (B as [k, n] at every depth that
+// the tile kernels take): no kernel is built for its other form.
 template <typename T, typename OUT_T, int MODE, typename CFG>
 int launch_pipe(const Problem& p, hipStream_t stream) {
   if (p.g.b_kn) return launch_pipe_kn<T, OUT_T, MODE, CFG, true>(p, stream);
-  return launch_pipe_kn<T, OUT_T, MODE, CFG, false>(p, stream);
+  if constexpr (MODE != kOutBf16ViaF16)
+    return launch_pipe_kn<T, OUT_T, MODE, CFG, false>(p, stream);
+  return no_kernel();
+}
+
+// launch(kn, add) with the form of a product as constants: B as [k, n], with an addend.
+// Kernels are built for the forms there are: accumulators are rounded first only with
+// an addend, the Gram iteration's last product is a left one, and left products without
+// an addend are its alone (float16).
+template <typename T, int MODE, typename LAUNCH>
+int with_form(const GemmArgs& g, LAUNCH launch) {
+  using Yes = std::true_type;
+  using No = std::false_type;
+  if (g.b_kn) {
+    if (g.d) return launch(Yes{}, Yes{});
+    if constexpr (std::is_same<T, _Float16>::value) return launch(Yes{}, No{});
+  } else if constexpr (MODE != kOutBf16ViaF16) {
+    if (g.d) return launch(No{}, Yes{});
+    if constexpr (MODE != kOutRoundAcc) return launch(No{}, No{});
+  }
+  return no_kernel();
 }
 
 template <typename T, typename OUT_T, int MODE, typename CFG, bool BKN, bool ADD>
@@ -1803,11 +1831,9 @@ int launch_tile_kn(const Problem& p, hipStream_t stream) {
 
 template <typename T, typename OUT_T, int MODE, typename CFG>
 int launch_tile(const Problem& p, hipStream_t stream) {
-  if (p.g.d)
-    return p.g.b_kn ? launch_tile_kn<T, OUT_T, MODE, CFG, true, true>(p, stream)
-                    : launch_tile_kn<T, OUT_T, MODE, CFG, false, true>(p, stream);
-  return p.g.b_kn ? launch_tile_kn<T, OUT_T, MODE, CFG, true, false>(p, stream)
-                  : launch_tile_kn<T, OUT_T, MODE, CFG, false, false>(p, stream);
+  return with_form<T, MODE>(p.g, [&](auto kn, auto add) {
+    return launch_tile_kn<T, OUT_T, MODE, CFG, decltype(kn)::value, decltype(add)::value>(p, stream);
+  });
 }
 
 // Workgroups a tile size yields (symmetric products: upper-triangle tiles).
@@ -1896,12 +1922,10 @@ int launch_tile_group_kn(const std::vector<const Problem*>& ps, hipStream_t stre
 
 template <typename T, typename OUT_T, int MODE, typename CFG>
 int launch_tile_group(const std::vector<const Problem*>& ps, hipStream_t stream) {
-  const bool kn = ps[0]->g.b_kn, add = ps[0]->g.d != nullptr;
-  if (add)
-    return kn ? launch_tile_group_kn<T, OUT_T, MODE, CFG, true, true>(ps, stream)
-              : launch_tile_group_kn<T, OUT_T, MODE, CFG, false, true>(ps, stream);
-  return kn ? launch_tile_group_kn<T, OUT_T, MODE, CFG, true, false>(ps, stream)
-            : launch_tile_group_kn<T, OUT_T, MODE, CFG, false, false>(ps, stream);
+  return with_form<T, MODE>(ps[0]->g, [&](auto kn, auto add) {
+    return launch_tile_group_kn<T, OUT_T, MODE, CFG, decltype(kn)::value, decltype(add)::value>(
+        ps, stream);
+  });
 }
 
 template <typename T, typename OUT_T, int MODE>
