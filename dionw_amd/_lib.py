@@ -188,7 +188,14 @@ def int64_array(values: Sequence[int]) -> ctypes.Array[ctypes.c_int64]:
 
 
 def stream_handle(device: torch.device | None = None) -> int:
-    """The raw HIP stream of torch's current stream on ``device``."""
+    """The raw HIP stream of torch's current stream on ``device``.
+
+    Raises:
+        ValueError: For a device that is no GPU, before anything is launched on its
+            tensors' addresses.
+    """
+    if device is not None and device.type != "cuda":
+        raise ValueError(f"the HIP kernels need GPU tensors, got tensors on {device}")
     index = None if device is None else device.index
     return int(torch._C._cuda_getCurrentRawStream(
         torch.cuda.current_device() if index is None else index))
