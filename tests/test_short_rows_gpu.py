@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from dionw_amd import _lib
+from dionw_amd.newton_schulz import _INPUT_ELEMS
 from oracle.dion_ref import row_l1_scores
 
 pytestmark = pytest.mark.gpu
@@ -54,3 +55,65 @@ def test_short_row_sums(rows: int, cols: int) -> None:
                   rowsq.data_ptr(), _lib.F32, stream)
         close(u)
         assert rowsq[-1] == -1
+
+
+def _extended(x: torch.Tensor, to: int) -> torch.Tensor:
+    """``x`` with zero columns appended: they change no sum, but rows past the short
+    ones' 1024 columns take the workgroup per row."""
+    out = torch.zeros(x.shape[0], to, dtype=x.dtype)
+    out[:, :x.shape[1]] = x
+    return out
+
+
+@pytest.mark.parametrize("elem", [_lib.F32, _lib.F16, _lib.BF16])
+@pytest.mark.parametrize("cols", [4, 64, 252, 256, 260, 508, 512, 768, 1020, 1024])
+def test_short_row_sums_have_the_bits_of_long_rows(cols: int, elem: int) -> None:
+    """Sums of squares of rows in a wave each, bit for bit those of the same rows in a
+    workgroup each: with scores, and alone with and without momentum, heavy ball and
+    Nesterov, rounded to bf16 first or not (``elem``: the iteration's type)."""
+    rows, mu = 37, 0.95
+    print(f"{rows}x{cols} {elem}", flush=True)
+    g = torch.Generator().manual_seed(cols)
+    grad, m0 = torch.randn(rows, cols, generator=g), torch.randn(rows, cols, generator=g)
+    stream = _lib.stream_handle(DEV)
+
+    def sums(width: int) -> list[torch.Tensor]:
+        x, m = (_extended(t, width).to(DEV) for t in (grad, m0))
+        out = []
+        for momentum, nesterov in ((None, 0), (m, 0), (m, 1)):
+            rowsq = torch.full((rows,), -1.0, device=DEV)
+            _lib.call("dionw_full_sumsq", _pointers([x]), 1, rows, width,
+                      None if momentum is None else momentum.data_ptr(), mu, nesterov,
+                      rowsq.data_ptr(), elem, stream)
+            out.append(rowsq)
+        scores, rowsq = (torch.full((rows,), -1.0, device=DEV) for _ in range(2))
+        _lib.call("dionw_accumulate_scores", _pointers([x]), 1, rows, width, m.data_ptr(),
+                  scores.data_ptr(), rowsq.data_ptr(), elem, stream)
+        return [*out, rowsq, scores]
+
+    for i, (short, long) in enumerate(zip(sums(cols), sums(2048), strict=True)):
+        assert torch.equal(short, long), f"pass {i}"
+
+
+@pytest.mark.parametrize("elem", [_lib.F16, _lib.BF16])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cols", [8, 260, 576, 1024])
+def test_short_rows_of_an_input_have_the_bits_of_long_rows(cols: int, dtype: torch.dtype,
+                                                           elem: int) -> None:
+    """The same for the row sums of ``dionw_normalize_input``, on each input type."""
+    rows = 13
+    print(f"{rows}x{cols} {dtype} {elem}", flush=True)
+    source = torch.randn(rows, cols, generator=torch.Generator().manual_seed(cols)).to(dtype)
+    stream = _lib.stream_handle(DEV)
+
+    def sums(width: int) -> torch.Tensor:
+        x = _extended(source, width).to(DEV)
+        rowsq, den = torch.full((rows,), -1.0, device=DEV), torch.zeros(1, device=DEV)
+        pad = (width + 7) // 8 * 8
+        out = torch.empty(16, pad, dtype=torch.int16, device=DEV)
+        _lib.call("dionw_normalize_input", x.data_ptr(), _INPUT_ELEMS[dtype], 1, rows, width, 1.0,
+                  1e-8, rowsq.data_ptr(), den.data_ptr(), 16, pad, elem, out.data_ptr(), None,
+                  stream)
+        return rowsq
+
+    assert torch.equal(sums(cols), sums(2048))
