@@ -833,6 +833,11 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
                                               unsigned char* smem) {
   constexpr int BM = CFG::BM, BN = CFG::BN, NT = CFG::threads, CH = BN / 8;
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  // 16 bytes of an output row that may start at any element: rows of no multiple of 8
+  // are stored like the others (the hardware takes unaligned stores whole). In stores of
+  // single elements / here, us: 11 x 1977^2 x 192 symmetric 100 / 41, 22 x 2223x264x128
+  // with its transpose 43 / 25, 199 x 2746x364x128 with its transpose 705 / 287.
+  typedef uint32_t u4any __attribute__((ext_vector_type(4), aligned(2)));
   typedef OUT_T o4 __attribute__((ext_vector_type(4)));
   typedef T t4 __attribute__((ext_vector_type(4)));
   const int wm = wave / CFG::WN, wn = wave % CFG::WN;
@@ -879,10 +884,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
     }
     __syncthreads();
   }
-  const bool vec_rows = (g.ldc % 8 == 0) && (g.sc % 8 == 0) &&
-                        ((reinterpret_cast<uintptr_t>(g.c) | reinterpret_cast<uintptr_t>(g.c_diag)) & 15) == 0;
-  const bool vec_cols = g.ldct % 8 == 0 && g.sct % 8 == 0 && (reinterpret_cast<uintptr_t>(g.ct) & 15) == 0;
-  if (m0 + BM <= g.m_lim && n0 + BN <= g.n_lim && vec_rows && vec_cols) {
+  if (m0 + BM <= g.m_lim && n0 + BN <= g.n_lim) {
     // A whole tile: every LDS read of a batch is issued before its first store. A
     // diagonal tile stores its 8x8 blocks on and above the diagonal as they lie and
     // those above it mirrored.
@@ -900,7 +902,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) {
           if (diag_tile && ch < ((r0 + (b + i) * STEP) >> 3)) continue;
-          if (C) *reinterpret_cast<u4*>(C + at + (int64_t)(i * STEP) * g.ldc) = v[i];
+          if (C) *reinterpret_cast<u4any*>(C + at + (int64_t)(i * STEP) * g.ldc) = v[i];
           if (CD) {
             const int r = r0 + (b + i) * STEP;
             if (diag_tile && ch == (r >> 3)) {
@@ -911,7 +913,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
                 if (e == (r & 7)) x[e] = (OUT_T)((float)x[e] + g.diag_shift);
               __builtin_memcpy(&v[i], x, 16);
             }
-            *reinterpret_cast<u4*>(CD + at + (int64_t)(i * STEP) * g.ldc) = v[i];
+            *reinterpret_cast<u4any*>(CD + at + (int64_t)(i * STEP) * g.ldc) = v[i];
           }
         }
       }
@@ -938,9 +940,9 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) {
           if (diag_tile && r8 >= ((c + i * CSTEP) & ~7)) continue;
-          *reinterpret_cast<u4*>(CT + (int64_t)(n0 + c + i * CSTEP) * g.ldct + m0 + r8) = v[i];
+          *reinterpret_cast<u4any*>(CT + (int64_t)(n0 + c + i * CSTEP) * g.ldct + m0 + r8) = v[i];
           if (g.sym && CD)
-            *reinterpret_cast<u4*>(CD + (int64_t)(n0 + c + i * CSTEP) * g.ldc + m0 + r8) = v[i];
+            *reinterpret_cast<u4any*>(CD + (int64_t)(n0 + c + i * CSTEP) * g.ldc + m0 + r8) = v[i];
         }
       }
     }
@@ -952,10 +954,10 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
       const int gr = m0 + r, gc = n0 + 8 * ch;
       if (gr >= g.m_lim || gc >= g.n_lim || (diag_tile && ch < (r >> 3))) continue;
       const OUT_T* src = tile + epi_off<BN>(r, ch);
-      if (gc + 8 <= g.n_lim && vec_rows && !(CD && gr >= gc && gr < gc + 8)) {
+      if (gc + 8 <= g.n_lim && !(CD && gr >= gc && gr < gc + 8)) {
         const u4 v = *reinterpret_cast<const u4*>(src);
-        if (C) *reinterpret_cast<u4*>(C + (int64_t)gr * g.ldc + gc) = v;
-        if (CD) *reinterpret_cast<u4*>(CD + (int64_t)gr * g.ldc + gc) = v;
+        if (C) *reinterpret_cast<u4any*>(C + (int64_t)gr * g.ldc + gc) = v;
+        if (CD) *reinterpret_cast<u4any*>(CD + (int64_t)gr * g.ldc + gc) = v;
       } else {
         for (int e = 0; e < 8; ++e) {
           const int c = gc + e;
@@ -980,11 +982,11 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, f32x4 (&acc)[CF
       OUT_T v[8];
       __builtin_memcpy(v, &lo, 8);
       __builtin_memcpy(v + 4, &hi, 8);
-      if (gr + 8 <= g.m_lim && vec_cols) {
+      if (gr + 8 <= g.m_lim) {
         u4 w;
         __builtin_memcpy(&w, v, 16);
-        *reinterpret_cast<u4*>(CT + (int64_t)gc * g.ldct + gr) = w;
-        if (g.sym && CD) *reinterpret_cast<u4*>(CD + (int64_t)gc * g.ldc + gr) = w;
+        *reinterpret_cast<u4any*>(CT + (int64_t)gc * g.ldct + gr) = w;
+        if (g.sym && CD) *reinterpret_cast<u4any*>(CD + (int64_t)gc * g.ldc + gr) = w;
       } else {
         for (int e = 0; e < 8; ++e) {
           if (gr + e >= g.m_lim) continue;

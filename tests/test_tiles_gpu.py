@@ -216,3 +216,37 @@ def test_many_thin_blocks_are_iterated_alike(rows: int, cols: int, kind) -> None
     got = f(x, 1e-8)
     for b in (0, 7, 255, 256, 299):
         assert torch.equal(got[b], f(x[b:b + 1], 1e-8)[0]), f"block {b}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize(("batch", "m", "n", "k", "symmetric"), [
+    (1, 64, 64, 64, False), (3, 65, 129, 192, False), (300, 64, 72, 64, False),  # 64x64 tiles
+    (40, 256, 257, 128, False), (40, 250, 250, 128, True),  # 128x128
+    (40, 512, 513, 128, False), (40, 512, 512, 192, True), (40, 515, 515, 128, True),  # 256x256
+])
+@pytest.mark.parametrize("offset", [1, 3, 4])
+def test_outputs_in_rows_that_start_anywhere(batch, m, n, k, symmetric, offset, dtype) -> None:
+    """Outputs whose rows start at any element have the bits of aligned ones, and nothing
+    beside them is written."""
+    print(f"{batch} x {m}x{n}x{k} symmetric {symmetric} offset {offset} {dtype}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a = _strided((batch, m, k), 0, dtype, g)
+    b = a if symmetric else _strided((batch, n, k), 8, dtype, g)
+
+    def outputs(rows: int, cols: int, start: int, pad: int) -> tuple[torch.Tensor, torch.Tensor]:
+        store = torch.full((start + batch * rows * (cols + pad) + 8,), 7.0, device=DEV, dtype=dtype)
+        whole = store[start:start + batch * rows * (cols + pad)].view(batch, rows, cols + pad)
+        return store, whole[:, :, :cols]
+
+    results = []
+    for start, pad in ((0, -n % 8 + 8), (offset, (-n % 8 + 8) + offset)):
+        store, out = outputs(m, n, start, pad)
+        store_t, out_t = outputs(n, m, start, (-m % 8 + 8) + (offset if start else 0))
+        gemm_nt(a, b, alpha=0.5, out=out, out_t=None if symmetric else out_t, symmetric=symmetric)
+        results.append(out.clone())
+        if not symmetric:
+            assert torch.equal(out_t, out.mT)
+        for written, s in ((out, store), (out_t, store_t)):
+            written.fill_(7.0)
+            assert (s == 7).all(), "wrote beside the rows"
+    assert torch.equal(*results)
