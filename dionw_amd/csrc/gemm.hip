@@ -1299,15 +1299,15 @@ __device__ __forceinline__ void quad_tile(const GemmArgs& g, int w) {
 // ---- 64x64 tiles -------------------------------------------------------------------
 //
 // For products of so few tiles that their time is one tile's chain of stages and the
-// launch: 4 waves of one 32x32 fragment each, and a ring of 8 stages (64 deep) per
+// launch, and for those of one stage: 4 waves of one 32x32 fragment each, and a ring of 8 stages (64 deep) per
 // workgroup, so that 7 stages are on their way from the first moment and a stage has
 // six others' time to land. A stage's fragments are read under the MFMAs of the stage
 // before; one barrier per stage. Measured in a chain of launches, us, against 128x128
 // tiles: 1024^3 symmetric with addend 12.1 / 8.7, 512^3 9.1 / 6.6, 256^3 7.4 / 5.9
 // (an empty kernel takes 4.7); a 1 x 1024x1024 Newton-Schulz call 249 / 147.
 // The ring has no more slots than the product has stages, so that the workgroups of a
-// one-stage product take 24 KB and share a CU: such products run these tiles whatever
-// their number. On 128x128 tiles / here, us: 1000 x 64^3 with addend 19.5 / 9.8, 3000 x
+// one-stage product take 24 KB and share a CU: such products may run these tiles whatever
+// their number (tile_fits). On 128x128 tiles / here, us: 1000 x 64^3 with addend 19.5 / 9.8, 3000 x
 // 64x256x64 117 / 58; Gram calls on 432 x 64x768 349 / 171, 455 x 48x192 292 / 124,
 // 16384 x 64x64 5370 / 1450. (A whole ring each takes 272 on the first of these calls.)
 struct SmallTile {
